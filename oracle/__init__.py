@@ -42,7 +42,7 @@ def build(ref: bool | None = None) -> None:
     """Compile liboracle.so (and the reference closure when its sources exist)."""
     targets = ["all"]
     if ref is None:
-        ref = os.path.isdir(REF_SRC)
+        ref = os.path.isfile(os.path.join(REF_SRC, "src", "lbm", "collision", "K17CompressibleNavierStokes.h"))
     if ref:
         targets.append("ref")
     subprocess.run(["make", "-s", "-C", HERE, f"-j{min(8, os.cpu_count() or 1)}"] + targets, check=True)
