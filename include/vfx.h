@@ -140,13 +140,14 @@ typedef struct vfx_lattice {
     double forces[3];
     double force_factor;
 
-    /* Launch shape of the collide-and-stream step: nodes per workgroup along
-     * x (structured step: 64, 128 or 256; 0 = 256; the sparse step's
-     * workgroups are 256 work items: 0 or 256) and the XCD tile run
+    /* Launch shape of the collide-and-stream step: nodes per workgroup
+     * (structured step: 64, 128 or 256 consecutive node numbers; 0 = the
+     * built-in choice, 128 for the default FP32 K17, else 256; the sparse
+     * step's workgroups are 256 work items: 0 or 256) and the XCD tile run
      * (workgroups reach the 8 XCDs round robin; consecutive tiles are handed
      * to each XCD in runs of this many, a power of two up to 4096, 1 = plain
-     * order; 0 = the built-in choice, 16 for 2- and 4-byte populations, 256
-     * for 8-byte ones).
+     * order; 0 = the built-in choice: structured step 4 for 2-byte
+     * populations, else 16; sparse step 16, 256 for 8-byte populations).
      * vfx_k17_autotune measures them.  Other kernels ignore both. */
     uint32_t tile_nodes;
     uint32_t xcd_run;

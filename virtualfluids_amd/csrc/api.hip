@@ -80,7 +80,9 @@ vfx_status make_lat(const vfx_lattice* in, vfx::Lat& L)
         L.ny = (uint32_t)ny;
         L.nz = (uint32_t)nz;
         L.chunks = (uint32_t)((nx + tile - 1) / tile);
-        L.tile = (uint32_t)tile;
+        L.tile = in->tile_nodes;
+        L.div_x = vfx::make_fastdiv(L.nx);
+        L.div_y = vfx::make_fastdiv(L.ny);
         L.solid = in->solid_mask;
     } else {
         if (!in->neighbor_x || !in->neighbor_y || !in->neighbor_z)

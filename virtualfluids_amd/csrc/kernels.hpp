@@ -99,11 +99,37 @@ template <> struct Buf<_Float16> {
 template <typename S> struct Compute { using T = float; };
 template <> struct Compute<double> { using T = double; };
 
+// Exact unsigned division by a run-time invariant d (Granlund & Montgomery,
+// "Division by invariant integers using multiplication", PLDI 1994, fig. 4.1):
+// l = ceil(log2 d), m = floor(2^32 (2^l - d) / d) + 1,
+// q = (t + ((n - t) >> 1)) >> (l - 1) with t = mulhi(m, n); d = 1 is passed
+// through.
+struct FastDiv {
+    uint32_t d, m, l;
+};
+inline FastDiv make_fastdiv(uint32_t d)
+{
+    FastDiv f{d, 0, 0};
+    if (d <= 1) return f;
+    uint32_t l = 0;
+    while ((1ull << l) < d) ++l;
+    f.l = l;
+    f.m = (uint32_t)((((1ull << l) - d) << 32) / d + 1);
+    return f;
+}
+__device__ __forceinline__ uint32_t fastdiv(uint32_t n, const FastDiv& f)
+{
+    if (f.d <= 1) return n;
+    const uint32_t t = __umulhi(f.m, n);
+    return (t + ((n - t) >> 1)) >> (f.l - 1);
+}
+
 // Device view of a vfx_lattice.
 struct Lat {
     void* f;
     uint64_t N;
-    uint32_t nx, ny, nz, chunks; // direct addressing; chunks = blocks per x row
+    uint32_t nx, ny, nz, chunks; // direct addressing; chunks = blocks per x row (k_step_fused)
+    FastDiv div_x, div_y;        // division by nx, ny
     const uint32_t* solid;
     const uint32_t* nbx;
     const uint32_t* nby;
@@ -124,7 +150,7 @@ struct Lat {
     double gforce[3];      // global force, unscaled
     double force_factor;
     uint32_t xrun_lg;      // 1 + log2 of the XCD tile run of the direct step (0: xcd_run<S>())
-    uint32_t tile;         // nodes per workgroup along x of the direct step
+    uint32_t tile;         // nodes per workgroup of the direct step (0: built-in)
     const uint4* rgroups;  // sparse: per 64 work items {base node, y stride, z stride, regular}, or NULL
 };
 
@@ -191,11 +217,23 @@ __device__ __forceinline__ void nbrs_interior(const Lat& L, uint32_t x, uint32_t
     kk[6] = kk[4] + sy;
     kk[7] = kk[6] + 1;
 }
+// node k of the box: its coordinates by two multiply-high divisions, the
+// others by adds of one x, y and z step (1, nx, nx ny, or back across the box)
 __device__ __forceinline__ void nbrs_direct(const Lat& L, uint32_t k, uint32_t (&kk)[8])
 {
-    const uint32_t x = k % L.nx;
-    const uint32_t r = k / L.nx;
-    nbrs_direct_xyz(L, x, r % L.ny, r / L.ny, kk);
+    const uint32_t r = fastdiv(k, L.div_x), z = fastdiv(r, L.div_y);
+    const uint32_t sz = L.nx * L.ny;
+    const uint32_t dx = k - r * L.nx + 1u == L.nx ? 1u - L.nx : 1u;
+    const uint32_t dy = r - z * L.ny + 1u == L.ny ? L.nx - sz : L.nx;
+    const uint32_t dz = z + 1u == L.nz ? sz - (uint32_t)L.N : sz;
+    kk[0] = k;
+    kk[1] = k + dx;
+    kk[2] = k + dy;
+    kk[3] = kk[1] + dy;
+    kk[4] = k + dz;
+    kk[5] = kk[1] + dz;
+    kk[6] = kk[2] + dz;
+    kk[7] = kk[3] + dz;
 }
 __device__ __forceinline__ void nbrs_sparse(const Lat& L, uint32_t k, uint32_t (&kk)[8])
 {
@@ -338,8 +376,9 @@ template <typename T> __device__ __forceinline__ void write_macro(const Lat& L, 
 // blocks x*C .. x*C+C-1 of each group (a tail shorter than 8C keeps the plain
 // order).  Shared lines inside a run meet in one L2.  Runs much longer than
 // this spread the XCDs over distant parts of each plane at once, which costs
-// more than it saves for the 2-byte form (measured on MI355X: 16 blocks for
-// 2- and 4-byte populations, 256 for 8-byte ones).
+// more than it saves for the 2-byte form.  xcd_run is the built-in run of the
+// row-mapped and sparse steps (k_step_fused, k_step_sparse), step_run that of
+// the structured step, whose tiles are consecutive node numbers.
 constexpr uint32_t kXcds = 8;
 __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t G, uint32_t C)
 {
@@ -347,6 +386,11 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t G, uint32_t C
     return b >= full ? b : (b / span) * span + (b % kXcds) * C + (b / kXcds) % C;
 }
 template <typename S> constexpr uint32_t xcd_run() { return sizeof(S) == 8 ? 256u : 16u; }
+// us per K17 step by run of 4 / 16 / 256 tiles of the built-in width (MI355X):
+// FP16 512x256x256 709 / 733 / 784, 230x171x125 96.1 / 98.8 / 97.6; FP32
+// 512x256x256 1360 / 1359 / 1437; FP64 256^3 1411 / 1434 / 1434, BGK 160^3
+// 362 / 348 / 357
+template <typename S> constexpr uint32_t step_run() { return sizeof(S) == 2 ? 4u : 16u; }
 // the same for a run of 2^lg tiles (shifts only)
 __device__ __forceinline__ uint32_t xcd_block_pow2(uint32_t b, uint32_t G, uint32_t lg)
 {
@@ -354,21 +398,27 @@ __device__ __forceinline__ uint32_t xcd_block_pow2(uint32_t b, uint32_t G, uint3
     return b >= full ? b : ((b >> sh) << sh) + ((b & (kXcds - 1u)) << lg) + ((b >> 3) & ((1u << lg) - 1u));
 }
 
-// Direct (structured) addressing: one block covers `blockDim.x` consecutive
-// nodes of one x row, so every row index below is wave-uniform (scalar ALU).
-// Block `block` of the lattice's `blocks`.
+// Direct (structured) addressing: a tile is blockDim.x consecutive node
+// numbers, whatever row they lie in.  The step is bound by its 27 in-place
+// plane streams, so what matters is that every wavefront has 64 nodes and that
+// its elements of a plane are one contiguous piece; a tile per x row leaves
+// lanes idle wherever nx is no multiple of 64 (66: half the wavefronts hold 2
+// nodes).  The price is a per-lane decode of the node (two multiply-high
+// divisions, ~20 instructions), hidden behind the loads.  Against a tile per
+// row, MI355X, us per step: FP64 66^3 36 -> 26, FP16 with AMD 224x144x120 195
+// -> 175, FP16 512x256x256 736 -> 700 (with step_run), FP32 230x171x125 218 ->
+// 207 (with 128-node tiles).
+// Tile `block` of the lattice's `blocks`.
 template <typename S, int COLL, bool EVEN, bool FAST>
 __device__ __forceinline__ void step_direct_body(const Lat& L, const Rates<typename Compute<S>::T>& R, uint32_t block,
                                                  uint32_t blocks)
 {
     using T = typename Compute<S>::T;
-    const uint32_t blk = L.xrun_lg ? xcd_block_pow2(block, blocks, L.xrun_lg - 1u) : xcd_block(block, blocks, xcd_run<S>());
-    const uint32_t row = blk / L.chunks;
-    const uint32_t x = (blk - row * L.chunks) * blockDim.x + threadIdx.x;
-    if (x >= L.nx) return;
-    const uint32_t y = row % L.ny, z = row / L.ny;
+    const uint32_t blk = L.xrun_lg ? xcd_block_pow2(block, blocks, L.xrun_lg - 1u) : xcd_block(block, blocks, step_run<S>());
+    const uint32_t k = blk * blockDim.x + threadIdx.x;
+    if (k >= (uint32_t)L.N) return;
     uint32_t kk[8];
-    nbrs_direct_xyz(L, x, y, z, kk);
+    nbrs_direct(L, k, kk);
     if (is_solid(L, kk[0])) return;
     T m[27], mv[4];
     constexpr bool O2 = FAST && coll_op(COLL) == VFX_K17 && coll_turb(COLL) == kTurbNone && sizeof(S) == 2;
@@ -2071,36 +2121,11 @@ __global__ void __launch_bounds__(256) k_step_levels(LevelPair<S> P)
 // lane-masked store.  The wall layer therefore holds stale values after a
 // step, which nothing reads.
 
-// Exact unsigned division by a run-time invariant d (Granlund & Montgomery,
-// "Division by invariant integers using multiplication", PLDI 1994, fig. 4.1):
-// l = ceil(log2 d), m = floor(2^32 (2^l - d) / d) + 1,
-// q = (t + ((n - t) >> 1)) >> (l - 1) with t = mulhi(m, n); d = 1 is passed
-// through.
-struct FastDiv {
-    uint32_t d, m, l;
-};
-inline FastDiv make_fastdiv(uint32_t d)
-{
-    FastDiv f{d, 0, 0};
-    if (d <= 1) return f;
-    uint32_t l = 0;
-    while ((1ull << l) < d) ++l;
-    f.l = l;
-    f.m = (uint32_t)((((1ull << l) - d) << 32) / d + 1);
-    return f;
-}
 // a value the caller knows to be uniform across the wavefront, as a scalar
 __device__ __forceinline__ uint32_t uni(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ uint64_t uni64(uint64_t v)
 {
     return (uint64_t)uni((uint32_t)v) | ((uint64_t)uni((uint32_t)(v >> 32)) << 32);
-}
-
-__device__ __forceinline__ uint32_t fastdiv(uint32_t n, const FastDiv& f)
-{
-    if (f.d <= 1) return n;
-    const uint32_t t = __umulhi(f.m, n);
-    return (t + ((n - t) >> 1)) >> (f.l - 1);
 }
 
 template <typename T> struct DomainDev {
@@ -2338,11 +2363,13 @@ inline unsigned grid_for(uint64_t n, int block) { return (unsigned)((n + block -
 
 // Occupancy cap of the structured step: LDS requested at launch and not
 // used, so that at most 160 KiB / cap workgroups share a CU.  The FP32
-// reduced-operation step (58 VGPRs, 8 waves per SIMD by registers) runs
-// fastest with at most 6 workgroups per CU (MI355X, 512x256x256, tuned launch
-// shapes: 1.33 ms per step against 1.40 uncapped; the tuner then picks
-// 128-node tiles, ~3 waves per SIMD); the sparse FP32 step with the same
-// cap 1.497 ms against 1.530.  The FP16 step is fastest at the 7
+// reduced-operation step (8 waves per SIMD by registers) runs fastest with at
+// most 6 workgroups of 128 nodes per CU, ~3 waves per SIMD: more of them in
+// flight only spread the 54 streams over more open pages (MI355X, us per step
+// by tiles of 64 / 128 / 256 nodes, each at most 6 per CU: 512x256x256 1559 /
+// 1359 / 1403, 230x171x125 215 / 207 / 216; 1404 without a cap); the sparse
+// FP32 step, whose workgroups are 256 work items, with the same cap 1497
+// against 1530.  The FP16 step is fastest at the 7
 // waves its registers allow (6 or 5 waves per SIMD measured slower), FP64 and
 // the reference-order kernels are limited by their registers; other
 // collision templates keep the uncapped launch.
@@ -2358,11 +2385,9 @@ template <typename S, int COLL, bool EVEN, bool FAST>
 hipError_t launch_step_t(const Lat& L, int direct, const Rates<typename Compute<S>::T>& R, hipStream_t st)
 {
     if (direct) {
-        const unsigned grid = L.chunks * L.ny * L.nz;
-        const unsigned block = (unsigned)((L.nx + L.chunks - 1) / L.chunks);
-        const unsigned b = block <= 64 ? 64 : block <= 128 ? 128 : 256;
-        hipLaunchKernelGGL((k_step_direct<S, COLL, EVEN, FAST>), dim3(grid), dim3(b), (step_lds_cap<S, COLL, FAST>()), st, L,
-                           R);
+        const unsigned tile = L.tile ? L.tile : step_lds_cap<S, COLL, FAST>() ? 128u : 256u;
+        hipLaunchKernelGGL((k_step_direct<S, COLL, EVEN, FAST>), dim3(grid_for(L.N, tile)), dim3(tile),
+                           (step_lds_cap<S, COLL, FAST>()), st, L, R);
     } else {
         const uint64_t n = node_items(L, 0);
         if (n == 0) return hipSuccess;
@@ -2475,9 +2500,8 @@ template <typename S> hipError_t launch_step_levels(const LevelInput* in, int n,
     uint32_t first = 0;
     for (int j = 0; j < n; ++j) {
         *L[j] = in[j].L;
-        L[j]->chunks = (L[j]->nx + tile - 1u) / tile; // blocks of `tile` nodes in this launch
         *R[j] = make_rates<T>(in[j].omega, in[j].lim, in[j].force, 0.0);
-        *blocks[j] = L[j]->chunks * L[j]->ny * L[j]->nz;
+        *blocks[j] = grid_for(L[j]->N, tile);
         if (j == 1) P.first1 = first;
         first += (*blocks[j] + kXcds - 1) / kXcds * kXcds;
     }
