@@ -1162,71 +1162,103 @@ template <typename T> __device__ __forceinline__ T proj(int d, T ux, T uy, T uz)
     return v;
 }
 
-// 6 w_d (c_d . u) with the component order VirtualFluids writes it
-// (VelocityBounceBack.cu:159-184); cpu_float reproduces BoundaryConditions.h:195-262
-// (float wall velocity, float component sum, double scale, float result).
-template <typename T>
-__device__ __forceinline__ T wall_term(int d, double ux, double uy, double uz, int cpu_float)
+// 6 w_d (c_d . u) as BoundaryConditions.h:195-262 rounds it (float wall
+// velocity, float component sum, double scale, float result)
+template <typename T> __device__ __forceinline__ T wall_term_cpu(int d, double ux, double uy, double uz)
 {
     const int n = weight_class(d);
     const double coef = n == 1 ? 4. / 9. : n == 2 ? 1. / 9. : 1. / 36.;
-    if (cpu_float) {
-        const float u[3] = {(float)ux, (float)uy, (float)uz};
-        const int c[3] = {cx(d), cy(d), cz(d)};
-        float s = 0.f;
-        bool first = true;
-        for (int a = 0; a < 3; ++a) {
-            if (c[a] == 0) continue;
-            if (first) { s = c[a] > 0 ? u[a] : -u[a]; first = false; }
-            else s = c[a] > 0 ? s + u[a] : s - u[a];
-        }
-        return (T)(double)(float)(coef * (double)s);
-    }
-    const T u[3] = {(T)ux, (T)uy, (T)uz};
-    const int c[3] = {cx(d), cy(d), cz(d)};
-    T s = T(0);
-    bool first = true;
-    for (int a = 0; a < 3; ++a) {
-        if (c[a] == 0) continue;
-        if (first) { s = c[a] > 0 ? u[a] : -u[a]; first = false; }
-        else s = c[a] > 0 ? s + u[a] : s - u[a];
-    }
-    return (T)coef * s;
+    const float s = proj<float>(d, (float)ux, (float)uy, (float)uz);
+    return (T)(double)(float)(coef * (double)s);
 }
 
 // Moving-wall halfway bounce-back (VelocityBounceBack_Device): for every wall
 // link d of a boundary node, the population leaving towards the wall comes back
 // as the opposite direction, minus the wall term.  Runs between the collision
 // of parity EVEN and the parity flip.
+//
+// fpost - 6 w_d (c_d . u): one explicit FMA in FP32, so that every kernel that
+// inlines it gives the same bits; product and difference rounded apart in FP64,
+// as the reference does
+template <typename T>
+__device__ __forceinline__ T bb_value(int d, T fpost, T ux, T uy, T uz, int cpu_float)
+{
+    if (cpu_float) return fpost - wall_term_cpu<T>(d, (double)ux, (double)uy, (double)uz);
+    const T coef = T(weight_class(d) == 1 ? 4. / 9. : weight_class(d) == 2 ? 1. / 9. : 1. / 36.);
+    const T s = proj<T>(d, ux, uy, uz);
+    if constexpr (sizeof(T) == 4) return __builtin_fmaf(-coef, s, fpost);
+    else return fpost - coef * s;
+}
+
+// Links D0 .. D0 + G - 1 (up to 26) of entry i: every fraction is loaded first,
+// then the populations of the wall links, then they are stored
+template <typename S, bool EVEN, int D0, int G>
+__device__ __forceinline__ void bb_links(const Lat& L, const BCDev& B, uint32_t i)
+{
+    using T = typename Compute<S>::T;
+    constexpr int D1 = D0 + G < 27 ? D0 + G : 27;
+    const uint32_t k = B.k[i];
+    bool on[G];
+    bool any = false;
+#pragma unroll
+    for (int d = D0; d < D1; ++d) {
+        const T q = bc_q<T>(B, d, i);
+        on[d - D0] = q >= T(0) && q <= T(1);
+        any |= on[d - D0];
+    }
+    if (!any || k >= L.N) return; // malformed list entry: never touch memory outside the lattice
+    uint32_t kk[8];
+    if (B.direct) nbrs_direct(L, k, kk);
+    else nbrs_sparse(L, k, kk);
+    T ux = B.vx ? bc_at<T>(B.vx, i) : T(0), uy = B.vy ? bc_at<T>(B.vy, i) : T(0), uz = B.vz ? bc_at<T>(B.vz, i) : T(0);
+    T f[G];
+#pragma unroll
+    for (int d = D0; d < D1; ++d) {
+        // post-collision population of direction d sits where e was read from
+        const int e = inv(d);
+        if (on[d - D0])
+            f[d - D0] = Storage<S, T>::ld(plane<S>(L, slot(e, EVEN)), kk[nbr(e)], L.ld[weight_class(d)], L.sh[d]);
+    }
+#pragma unroll
+    for (int d = D0; d < D1; ++d) {
+        // next step (parity !EVEN) reads direction e of node k from here
+        const int e = inv(d);
+        if (on[d - D0])
+            Storage<S, T>::st(plane<S>(L, slot(e, !EVEN)), kk[nbr(e)], bb_value<T>(d, f[d - D0], ux, uy, uz, B.cpu_float),
+                              L.st[weight_class(e)], L.ss[e]);
+    }
+}
 template <typename S, bool EVEN>
 __device__ __forceinline__ void bc_velocity_bb_entry(const Lat& L, const BCDev& B, uint32_t i)
 {
-    using T = typename Compute<S>::T;
-    if (i >= B.n) return;
-    uint32_t kk[8];
-    const uint32_t k = B.k[i];
-    if (k >= L.N) return; // malformed list entry: never touch memory outside the lattice
-    if (B.direct) nbrs_direct(L, k, kk);
-    else nbrs_sparse(L, k, kk);
-    const double ux = B.vx ? (double)bc_at<T>(B.vx, i) : 0.0, uy = B.vy ? (double)bc_at<T>(B.vy, i) : 0.0,
-                 uz = B.vz ? (double)bc_at<T>(B.vz, i) : 0.0;
-#pragma unroll
-    for (int d = 1; d < 27; ++d) {
-        const T q = bc_q<T>(B, d, i);
-        if (!(q >= T(0) && q <= T(1))) continue;
-        const int e = inv(d);
-        // post-collision population of direction d sits where e was read from
-        const T fpost = Storage<S, T>::ld(plane<S>(L, slot(e, EVEN)), kk[nbr(e)], L.ld[weight_class(d)], L.sh[d]);
-        const T v = fpost - wall_term<T>(d, ux, uy, uz, B.cpu_float);
-        // next step (parity !EVEN) reads direction e of node k from here
-        Storage<S, T>::st(plane<S>(L, slot(e, !EVEN)), kk[nbr(e)], v, L.st[weight_class(e)], L.ss[e]);
-    }
+    if (i < B.n) bb_links<S, EVEN, 1, 26>(L, B, i);
 }
 
+// One thread per link: blockIdx.y is the direction, so a wavefront holds one
+// direction of 64 boundary nodes and everything about the link is a constant of
+// the switch branch it takes.  Short lists are bound by latency: with the links
+// of a node one after another in one thread each waited for the one before (its
+// fraction, its population and its store, 26 round trips); here the chain is
+// fraction -> population -> store.  Long lists are bound by the cache lines of
+// faces normal to x, one per element.  MI355X, us per launch, before -> now:
+// cavity 30^3 FP32 13.6 -> 3.6, 64^3 FP64 17.5 -> 6.2, y and z walls and spheres
+// of a 320x130x134 sparse box FP16 33.9 -> 31.0; 3, 7, 13 and 26 links per
+// thread: 30^3 4.3 / 4.7 / 5.8 / 7.3, 128^3 FP16 14.4 / 14.9 / 14.9 / 15.9
+// against 15.9.
 template <typename S, bool EVEN>
 __global__ void __launch_bounds__(256) k_bc_velocity_bb(Lat L, BCDev B)
 {
-    bc_velocity_bb_entry<S, EVEN>(L, B, blockIdx.x * blockDim.x + threadIdx.x);
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= B.n) return;
+#define VFX_LINK(D) \
+    case D: bb_links<S, EVEN, D, 1>(L, B, i); break;
+    switch (blockIdx.y + 1) {
+        VFX_LINK(1) VFX_LINK(2) VFX_LINK(3) VFX_LINK(4) VFX_LINK(5) VFX_LINK(6) VFX_LINK(7) VFX_LINK(8) VFX_LINK(9)
+        VFX_LINK(10) VFX_LINK(11) VFX_LINK(12) VFX_LINK(13) VFX_LINK(14) VFX_LINK(15) VFX_LINK(16) VFX_LINK(17)
+        VFX_LINK(18) VFX_LINK(19) VFX_LINK(20) VFX_LINK(21) VFX_LINK(22) VFX_LINK(23) VFX_LINK(24) VFX_LINK(25)
+        VFX_LINK(26)
+    }
+#undef VFX_LINK
 }
 
 // Interpolated bounce-back family (NoSlipInterpolatedCompressible.cu:44-378,
@@ -2688,8 +2720,8 @@ template <typename S> hipError_t launch_bc(const Lat& L, const BCDev& B, int kin
     const dim3 g(grid_for(B.n, kBlock)), b(kBlock);
     switch (kind) {
     case VFX_BC_VELOCITY_BOUNCE_BACK:
-        if (even) hipLaunchKernelGGL((k_bc_velocity_bb<S, true>), g, b, 0, st, L, B);
-        else hipLaunchKernelGGL((k_bc_velocity_bb<S, false>), g, b, 0, st, L, B);
+        if (even) hipLaunchKernelGGL((k_bc_velocity_bb<S, true>), dim3(g.x, 26), b, 0, st, L, B);
+        else hipLaunchKernelGGL((k_bc_velocity_bb<S, false>), dim3(g.x, 26), b, 0, st, L, B);
         break;
     case VFX_BC_NOSLIP_INTERPOLATED:
         if (even) hipLaunchKernelGGL((k_bc_interp<S, true, VFX_BC_NOSLIP_INTERPOLATED>), g, b, 0, st, L, B);
