@@ -119,8 +119,9 @@ typedef struct vfx_lattice {
      * velocity gradients back into turbulent_viscosity
      * (K17CompressibleNavierStokes.h:355-368); VFX_TURB_AMD takes nu_t from
      * vfx_turbulent_viscosity_amd and makes the collision write rho/vx/vy/vz,
-     * which must then be set.  The reference-order K17 kernel runs (any
-     * kernel_variant).  BGK ignores the model. */
+     * which must then be set.  FP16 storage runs the reduced-operation K17
+     * (kernel_variant 0), FP32 and FP64 the reference order in every variant.
+     * BGK ignores the model. */
     int32_t turbulence_model;     /* vfx_turbulence_model */
     double sgs_constant;          /* Parameter::SGSConstant (Smagorinsky Cs, QR / AMD constant) */
     void* turbulent_viscosity;    /* n_nodes values, double for VFX_FP64 else float (Parameter turbViscosity) */

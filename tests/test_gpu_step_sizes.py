@@ -4,6 +4,7 @@ The sizes sit at the edges of the flat node mapping (one node in a direction,
 rows of one node more or less than a wavefront, a last tile of one node)."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 import virtualfluids_amd as vfx
@@ -25,3 +26,44 @@ def test_box_sizes_bitwise_in_fp64(cuda, dims, collision):
     st.step(3)
     ref = oracle.run(F0, dims, 3, 1.85, collision=collision)
     assert np.array_equal(st.populations().cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("model", ["smagorinsky", "qr", "amd"])
+@pytest.mark.parametrize("sparse", [False, True])
+def test_fp16_models_reduced_form_equals_the_reference_order(cuda, model, sparse):
+    """FP16 storage runs the reduced-operation K17 with the node's own rates,
+    variant="plain" the reference order: one step differs by the FP32 rounding
+    of ~1500 operations (1e-5 of the largest population, generous) plus one unit
+    of the half it is stored in (2^-10 of the population itself).  The eddy
+    viscosity is compared with FP64's from the same populations: the reduced
+    form is at most half as far off again as the reference order."""
+    print(f"[fp16 {model} {sparse}]", flush=True)
+    dims = (37, 11, 8)
+    n = int(np.prod(dims))
+    fields = cases.random_flow(dims, seed=4)
+    nut = 1e-3 * (1.0 + np.sin(np.arange(n)))
+    out = []
+    for storage, variant in (("fp16", "default"), ("fp16", "plain"), ("fp64", "default")):
+        kw = dict(storage=storage, omega=1.97, turbulence=model, sgs_constant=0.2, variant=variant)
+        if sparse:
+            k = np.arange(n)
+            x, y, z = k % dims[0], k // dims[0] % dims[1], k // (dims[0] * dims[1])
+
+            def at(a, b, c):
+                return (a % dims[0] + dims[0] * (b % dims[1] + dims[1] * (c % dims[2]))).astype(np.uint32)
+            lat = vfx.Lattice(neighbors=(at(x + 1, y, z), at(x, y + 1, z), at(x, y, z + 1)),
+                              node_types=np.full(n, 19, np.uint32), neighbor_inverse=at(x - 1, y - 1, z - 1), **kw)
+        else:
+            lat = vfx.Lattice(dims, **kw)
+        if storage == "fp16":
+            lat.init_equilibrium(*fields)
+            start = lat.read_populations()
+        else:
+            lat.write_populations(start)
+        lat.nut.copy_(torch.from_numpy(nut).to(lat.nut.dtype))
+        vfx.Stepper(lat, "k17").step(1)
+        out.append((lat.f.double().cpu().numpy().reshape(27, n), lat.nut.double().cpu().numpy()))
+    (a, va), (b, vb), (_, v) = out
+    assert np.all(np.abs(a - b) <= 1e-5 * np.abs(b).max(axis=1, keepdims=True) + 2.0 ** -10 * np.abs(b))
+    assert np.linalg.norm(va - v) <= 1.5 * np.linalg.norm(vb - v)
+    assert not np.array_equal(a, b)  # the two forms did run

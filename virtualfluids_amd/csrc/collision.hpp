@@ -550,14 +550,40 @@ __device__ __forceinline__ void bwdf2(float& a, float& b, float& c, float k, flo
     c = r2;
 }
 
+// The folded constants of a node that relaxes with omega / (1 + 3 omega nu_t).
+// (1/w - 1/2) factorA = (2 - w) (4 + 2 w - 3 w^2) / (2 w D) and (1/w - 1/2)
+// factorB = (2 - w) (4 + 28 w - 14 w^2) / (6 w D), D = 2 - 7 w + 5 w^2: one
+// reciprocal for both, and 2 - w is exact where 1/w - 1/2 cancels.
+__device__ __forceinline__ void node_rates(const Rates<float>& R0, float nut, Rates<float>& r)
+{
+    const float w = R0.omega / (1.f + 3.f * R0.omega * nut), w2 = w * w, tw = 2.f - w;
+    const float oPP = -8.f * tw * (1.f + 2.f * w) * rcpf(-8.f - 14.f * w + 7.f * w2);
+    const float oMM = -8.f * tw * (4.f * w - 7.f) * rcpf(56.f - 50.f * w + 9.f * w2);
+    const float oD = -24.f * tw * (-2.f - 7.f * w + 3.f * w2) * rcpf(48.f + 152.f * w - 130.f * w2 + 29.f * w2 * w);
+    const float h = tw * rcpf(w * (2.f - 7.f * w + 5.f * w2));
+    r = R0;
+    r.omega = w;
+    r.om1 = 1.f - w;
+    r.c3 = 3.f - 1.5f * w;
+    r.limP1 = R0.limP - oPP * R0.limP;
+    r.limM1 = R0.limM - oMM * R0.limM;
+    r.limD1 = R0.limD - oD * R0.limD;
+    r.A4 = h * (1.f / 3.f) * (4.f + 2.f * w - 3.f * w2);
+    r.B4 = h * (1.f / 18.f) * (4.f + 28.f * w - 14.f * w2);
+}
+
 #define VFX_M(a, b, c) m[cube(a, b, c)]
 
 // OUTER2: run the backward sweeps with bwdf2, so that population d leaves
 // scaled by 2^weight_class(d) (the caller's store removes the factor; used
 // where the store multiplies by a scale anyway, i.e. FP16 storage).
-template <bool OUTER2>
-__device__ __forceinline__ void k17_fast(float (&m)[27], const Rates<float>& R, float (&mv)[4])
+// TM: eddy-viscosity model; the node's rates then come from its own omega.
+template <bool OUTER2, int TM = kTurbNone>
+__device__ __forceinline__ void k17_fast(float (&m)[27], const Rates<float>& R0, float (&mv)[4], float& nut)
 {
+    Rates<float> Rt;
+    if constexpr (TM != kTurbNone) node_rates(R0, nut, Rt);
+    const Rates<float>& R = TM != kTurbNone ? Rt : R0;
     constexpr float c1o3 = 1.f / 3.f, c1o9 = 1.f / 9.f, c1o27 = 1.f / 27.f, c2o3 = 2.f / 3.f;
     // ---- macroscopic values from the sums the sweeps form anyway.  Per (x,y)
     // row of the z sweep: s = f(z-) + f(z+), d = f(z+) - f(z-), m0 = s + f(z0).
@@ -641,6 +667,8 @@ __device__ __forceinline__ void k17_fast(float (&m)[27], const Rates<float>& R, 
     const float dxux = -0.5f * omega * (mxxMyy + mxxMzz) + 0.5f * (m000 - mxxPyyPzz);
     const float dyuy = dxux + 1.5f * omega * mxxMyy;
     const float dzuz = dxux + 1.5f * omega * mxxMzz;
+    if constexpr (TM == kTurbSmagorinsky) nut = turbulent_viscosity_smagorinsky<float>(R.sgs, dxux, dyuy, dzuz, Dxy, Dxz, Dyz);
+    if constexpr (TM == kTurbQR) nut = turbulent_viscosity_qr<float>(R.sgs, dxux, dyuy, dzuz, Dxy, Dxz, Dyz);
     mxxPyyPzz = m000 - 1.5f * (vx2 * dxux + vy2 * dyuy + vz2 * dzuz);
     mxxMyy = R.om1 * mxxMyy - R.c3 * (vx2 * dxux - vy2 * dyuy);
     mxxMzz = R.om1 * mxxMzz - R.c3 * (vx2 * dxux - vz2 * dzuz);

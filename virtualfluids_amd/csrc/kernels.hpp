@@ -339,7 +339,7 @@ template <typename T, int COLL, bool FAST, bool OUTER2 = false>
 __device__ __forceinline__ void collide(T (&m)[27], const Rates<T>& R, T (&mv)[4], T& nut)
 {
     if constexpr (coll_op(COLL) == VFX_K17) {
-        if constexpr (FAST && sizeof(T) == 4 && coll_turb(COLL) == kTurbNone) k17_fast<OUTER2>(m, R, mv);
+        if constexpr (FAST && sizeof(T) == 4) k17_fast<OUTER2, coll_turb(COLL)>(m, R, mv, nut);
         else k17<T, coll_turb(COLL)>(m, R, mv, nut);
     } else {
         bgk<T>(m, R.omega, mv);
@@ -397,7 +397,6 @@ __device__ __forceinline__ uint32_t xcd_block_pow2(uint32_t b, uint32_t G, uint3
     const uint32_t sh = lg + 3u, full = (G >> sh) << sh;
     return b >= full ? b : ((b >> sh) << sh) + ((b & (kXcds - 1u)) << lg) + ((b >> 3) & ((1u << lg) - 1u));
 }
-
 // Direct (structured) addressing: a tile is blockDim.x consecutive node
 // numbers, whatever row they lie in.  The step is bound by its 27 in-place
 // plane streams, so what matters is that every wavefront has 64 nodes and that
@@ -421,7 +420,7 @@ __device__ __forceinline__ void step_direct_body(const Lat& L, const Rates<typen
     nbrs_direct(L, k, kk);
     if (is_solid(L, kk[0])) return;
     T m[27], mv[4];
-    constexpr bool O2 = FAST && coll_op(COLL) == VFX_K17 && coll_turb(COLL) == kTurbNone && sizeof(S) == 2;
+    constexpr bool O2 = FAST && coll_op(COLL) == VFX_K17 && sizeof(S) == 2;
     T nut = load_nut<T, COLL>(L, kk[0]);
     Rates<T> Rn;
     node_force<T, COLL>(L, kk[0], R, Rn);
@@ -561,7 +560,7 @@ __global__ void __launch_bounds__(256) k_step_sparse(Lat L, Rates<typename Compu
     }
     if (!active) return;
     T m[27], mv[4];
-    constexpr bool O2 = FAST && coll_op(COLL) == VFX_K17 && coll_turb(COLL) == kTurbNone && sizeof(S) == 2;
+    constexpr bool O2 = FAST && coll_op(COLL) == VFX_K17 && sizeof(S) == 2;
     T nut = load_nut<T, COLL>(L, kk[0]);
     Rates<T> Rn;
     node_force<T, COLL>(L, kk[0], R, Rn);
@@ -2429,15 +2428,30 @@ hipError_t launch_step_t(const Lat& L, int direct, const Rates<typename Compute<
     return hipGetLastError();
 }
 
+// The reduced-operation form (FP32 arithmetic only) or the reference order.
+// With an eddy-viscosity model the reduced form runs on 2-byte storage only: the
+// reference order (rates of every node with IEEE divisions, ~1500 instructions)
+// is bound by its arithmetic there, the reduced one by memory (MI355X,
+// 224x144x120 with AMD: 175 -> 105 us per step, 810 -> 541 per 4 steps with the
+// viscosity kernel), and both sit at the storage's rounding (error of the
+// populations against 64 bits after 10 steps 3.0e-4 to 4.3e-4, equal to 0.3%,
+// omega 1.8 to 1.999, all models).  On 4-byte storage both are bound by memory
+// (256x160x100: 185 us) and the reduced form's error is up to twice the
+// reference order's (8.3e-7 against 4.4e-7), so that one keeps the latter.
 template <typename S, int COLL>
-hipError_t launch_step_p(const Lat& L, int direct, bool even, const Rates<typename Compute<S>::T>& R, hipStream_t st)
+hipError_t launch_step_p(const Lat& L, int direct, bool even, bool fast, const Rates<typename Compute<S>::T>& R,
+                         hipStream_t st)
 {
+    if constexpr (coll_op(COLL) == VFX_K17 && (sizeof(S) == 2 || (sizeof(S) == 4 && coll_turb(COLL) == kTurbNone))) {
+        if (fast) return even ? launch_step_t<S, COLL, true, true>(L, direct, R, st)
+                              : launch_step_t<S, COLL, false, true>(L, direct, R, st);
+    }
     return even ? launch_step_t<S, COLL, true, false>(L, direct, R, st)
                 : launch_step_t<S, COLL, false, false>(L, direct, R, st);
 }
 
 // variant: 0 = default (FP64: reference operation order; FP32/FP16: reduced form), 1 = reference order;
-// turb: TurbModel of the K17 collision (reference operation order in every variant)
+// turb: TurbModel of the K17 collision
 template <typename S> hipError_t launch_step(const Lat& L, int direct, int coll, bool even, int variant, double omega,
                                              const double* lim, const double* force, int turb, double sgs,
                                              hipStream_t st)
@@ -2448,33 +2462,20 @@ template <typename S> hipError_t launch_step(const Lat& L, int direct, int coll,
     coll &= 15;
     const bool fast = sizeof(T) == 4 && variant == 0 && coll == VFX_K17;
     constexpr int K = VFX_K17, BF = kCollBodyForce;
-    if (coll == VFX_K17 && turb != kTurbNone) {
-        switch (turb) {
-        case kTurbSmagorinsky:
-            return bf ? launch_step_p<S, K | (kTurbSmagorinsky << 4) | BF>(L, direct, even, R, st)
-                      : launch_step_p<S, K | (kTurbSmagorinsky << 4)>(L, direct, even, R, st);
-        case kTurbAMD:
-            return bf ? launch_step_p<S, K | (kTurbAMD << 4) | BF>(L, direct, even, R, st)
-                      : launch_step_p<S, K | (kTurbAMD << 4)>(L, direct, even, R, st);
+#define VFX_TURB(TM) \
+    case TM: \
+        return bf ? launch_step_p<S, K | ((TM) << 4) | BF>(L, direct, even, fast, R, st) \
+                  : launch_step_p<S, K | ((TM) << 4)>(L, direct, even, fast, R, st)
+    if (coll == VFX_K17) switch (turb) {
+            VFX_TURB(kTurbSmagorinsky);
+            VFX_TURB(kTurbAMD);
+            VFX_TURB(kTurbQR);
         default:
-            return bf ? launch_step_p<S, K | (kTurbQR << 4) | BF>(L, direct, even, R, st)
-                      : launch_step_p<S, K | (kTurbQR << 4)>(L, direct, even, R, st);
+            return bf ? launch_step_p<S, K | BF>(L, direct, even, fast, R, st)
+                      : launch_step_p<S, K>(L, direct, even, fast, R, st);
         }
-    }
-    if (coll == VFX_K17 && bf) {
-        if (fast) return even ? launch_step_t<S, K | BF, true, true>(L, direct, R, st)
-                              : launch_step_t<S, K | BF, false, true>(L, direct, R, st);
-        return even ? launch_step_t<S, K | BF, true, false>(L, direct, R, st)
-                    : launch_step_t<S, K | BF, false, false>(L, direct, R, st);
-    }
-    if (coll == VFX_K17) {
-        if (fast) return even ? launch_step_t<S, VFX_K17, true, true>(L, direct, R, st)
-                              : launch_step_t<S, VFX_K17, false, true>(L, direct, R, st);
-        return even ? launch_step_t<S, VFX_K17, true, false>(L, direct, R, st)
-                    : launch_step_t<S, VFX_K17, false, false>(L, direct, R, st);
-    }
-    return even ? launch_step_t<S, VFX_BGK, true, false>(L, direct, R, st)
-                : launch_step_t<S, VFX_BGK, false, false>(L, direct, R, st);
+#undef VFX_TURB
+    return launch_step_p<S, VFX_BGK>(L, direct, even, false, R, st);
 }
 
 // K17 collide-and-stream of a structured lattice with fused boundary groups
