@@ -397,6 +397,10 @@ __device__ __forceinline__ uint32_t xcd_block_pow2(uint32_t b, uint32_t G, uint3
     const uint32_t sh = lg + 3u, full = (G >> sh) << sh;
     return b >= full ? b : ((b >> sh) << sh) + ((b & (kXcds - 1u)) << lg) + ((b >> 3) & ((1u << lg) - 1u));
 }
+// one contiguous eighth of the blocks per XCD (a grid of a multiple of 8 blocks):
+// stencils find their y and z neighbours' lines in the L2 they were read into
+__device__ __forceinline__ uint32_t xcd_slab(uint32_t b, uint32_t G) { return (b % kXcds) * (G / kXcds) + b / kXcds; }
+
 // Direct (structured) addressing: a tile is blockDim.x consecutive node
 // numbers, whatever row they lie in.  The step is bound by its 27 in-place
 // plane streams, so what matters is that every wavefront has 64 nodes and that
@@ -2327,32 +2331,41 @@ __device__ __forceinline__ void amd_derivatives(uint32_t k, uint32_t km, uint32_
                                                 const T* vy, const T* vz, T& dvx, T& dvy, T& dvz)
 {
     const T div = (fm && fp) ? T(0.5) : T(1);
-    dvx = ((fp ? vx[kp] : vx[k]) - (fm ? vx[km] : vx[k])) * div;
-    dvy = ((fp ? vy[kp] : vy[k]) - (fm ? vy[km] : vy[k])) * div;
-    dvz = ((fp ? vz[kp] : vz[k]) - (fm ? vz[km] : vz[k])) * div;
+    kp = fp ? kp : k;
+    km = fm ? km : k;
+    dvx = (elem(vx, kp) - elem(vx, km)) * div;
+    dvy = (elem(vy, kp) - elem(vy, km)) * div;
+    dvz = (elem(vz, kp) - elem(vz, km)) * div;
 }
 
+// Bound by its reads past L2: with the blocks round robin over the XCDs the rows
+// above, below, before and behind a block were in other L2s and came from memory
+// again, five times the fields' bytes.  With a contiguous eighth of the lattice
+// per XCD (xcd_slab) they are in its own: 224x144x120 33.6 -> 22.0 us (MI355X;
+// 62 MB that it must move, 12 us).  Selecting a neighbour by its index, once for
+// the three components, and 32-bit element offsets alone changed nothing.
 template <typename T> __global__ void __launch_bounds__(256) k_turb_amd(Lat L, int direct, T C)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= L.N) return;
-    const uint32_t k = (uint32_t)i;
+    const uint32_t k = xcd_slab(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    if (k >= (uint32_t)L.N) return;
     uint32_t kp[3], km[3];
-    bool fp[3], fm[3];
+    bool fp[3] = {true, true, true}, fm[3] = {true, true, true};
     if (direct) {
-        if (is_solid(L, k)) return;
-        const uint32_t x = k % L.nx, r = k / L.nx, y = r % L.ny, z = r / L.ny;
-        const uint32_t sy = L.nx, sz = L.nx * L.ny;
-        kp[0] = x + 1 == L.nx ? k - x : k + 1;
-        km[0] = x == 0 ? k + L.nx - 1 : k - 1;
-        kp[1] = y + 1 == L.ny ? k - y * sy : k + sy;
-        km[1] = y == 0 ? k + (L.ny - 1) * sy : k - sy;
-        kp[2] = z + 1 == L.nz ? k - z * sz : k + sz;
-        km[2] = z == 0 ? k + (L.nz - 1) * sz : k - sz;
+        const uint32_t r = fastdiv(k, L.div_x), x = k - r * L.nx, z = fastdiv(r, L.div_y), y = r - z * L.ny;
+        const uint32_t sy = L.nx, sz = L.nx * L.ny, n = (uint32_t)L.N;
+        kp[0] = k + (x + 1u == L.nx ? 1u - sy : 1u);
+        km[0] = k - (x == 0u ? 1u - sy : 1u);
+        kp[1] = k + (y + 1u == L.ny ? sy - sz : sy);
+        km[1] = k - (y == 0u ? sy - sz : sy);
+        kp[2] = k + (z + 1u == L.nz ? sz - n : sz);
+        km[2] = k - (z == 0u ? sz - n : sz);
+        if (L.solid) {
+            if (is_solid(L, k)) return;
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            fp[a] = !is_solid(L, kp[a]);
-            fm[a] = !is_solid(L, km[a]);
+            for (int a = 0; a < 3; ++a) {
+                fp[a] = !is_solid(L, kp[a]);
+                fm[a] = !is_solid(L, km[a]);
+            }
         }
     } else {
         if (L.types[k] != kGeoFluid) return;
@@ -2391,6 +2404,8 @@ template <typename T> __global__ void __launch_bounds__(256) k_turb_amd(Lat L, i
 constexpr int kBlock = 256;
 
 inline unsigned grid_for(uint64_t n, int block) { return (unsigned)((n + block - 1) / block); }
+// blocks of kBlock items, a multiple of 8 of them (xcd_slab)
+inline unsigned grid_slabs(uint64_t n) { return (grid_for(n, kBlock) + kXcds - 1) / kXcds * kXcds; }
 
 // Occupancy cap of the structured step: LDS requested at launch and not
 // used, so that at most 160 KiB / cap workgroups share a CU.  The FP32
@@ -2562,7 +2577,7 @@ inline hipError_t launch_sparse_groups(const Lat& L, uint4* table, uint32_t ngro
 template <typename S> hipError_t launch_turb_amd(const Lat& L, int direct, double sgs, hipStream_t st)
 {
     using T = typename Compute<S>::T;
-    hipLaunchKernelGGL((k_turb_amd<T>), dim3(grid_for(L.N, kBlock)), dim3(kBlock), 0, st, L, direct, (T)sgs);
+    hipLaunchKernelGGL((k_turb_amd<T>), dim3(grid_slabs(L.N)), dim3(kBlock), 0, st, L, direct, (T)sgs);
     return hipGetLastError();
 }
 
