@@ -300,10 +300,8 @@ vfx_status vfx_sparse_regular_groups(const vfx_lattice* lat, void* table, uint64
 vfx_status vfx_k17_autotune(const vfx_lattice* lat, int32_t is_even_timestep, int32_t collision_template,
                             int32_t steps, vfx_stream stream, uint32_t* tile_nodes, uint32_t* xcd_run, float* ms);
 
-/* Boundary conditions fused into the collide-and-stream kernel of a
- * structured lattice, so a boundary node's populations are not read again by
- * a kernel of their own (on a face normal to x each of them sits in its own
- * cache line).  node_mask: ceil(n_nodes/32) words, bit k set iff node k is an
+/* Boundary conditions of a structured lattice taken along with its
+ * collide-and-stream step.  node_mask: ceil(n_nodes/32) words, bit k set iff node k is an
  * entry of bc; word_base: ceil(n_nodes/32) words, the number of entries on
  * nodes below 32*w.  bc->k must be sorted ascending, one entry per node. */
 typedef struct vfx_fused_bc {
@@ -314,25 +312,25 @@ typedef struct vfx_fused_bc {
 
 /* vfx_k17_step (VFX_TEMPLATE_DEFAULT, default kernel variant, no turbulence
  * model) of a structured lattice with fused boundary conditions:
- *  - post[0..n_post-1] (n_post <= 2): interpolated kinds 1, 2, 3, 5, applied by
- *    the thread that collided each boundary node -- the same populations as
- *    vfx_bc_apply after the step;
+ *  - post[0..n_post-1] (n_post <= 2): interpolated kinds 1, 2, 3, 5, applied after
+ *    the step in this order, by the kernels of vfx_bc_apply (inside the step
+ *    they cost more than their own launches);
  *  - pre (or NULL): VFX_BC_PRESSURE_NEQ with normal dP00 (dM00) whose every
  *    entry has k_neighbor = k - 1 (k + 1) in the same wavefront of 64 nodes,
  *    i.e. x mod 64 != 0 (!= 63): the replacement vfx_bc_apply makes after the
  *    previous step's parity flip is made inside this step, from the
- *    neighbour's populations the neighbouring lane gathers (apply_pre = 1;
+ *    neighbour's populations the neighbouring lane gathers, which spares the
+ *    cache lines a kernel of its own reads again (where nx is no multiple of
+ *    64, a small launch before the step takes the nodes whose neighbour lies in
+ *    another 64 consecutive node numbers) (apply_pre = 1;
  *    0 on the first step of a run, before which no pressure boundary ran).
  *    Until the next step the boundary nodes then hold the un-replaced
  *    populations: vfx_bc_apply(pre->bc) with the new parity gives the state
  *    the separate launches leave, before it is read;
  *  - any_mask (or NULL): ceil(n_nodes/32) words, bit k set iff node k is an
- *    entry of some group above; loaded with the populations, it spares the
- *    other nodes the look-up in each group's mask.
+ *    entry of some group above (not read).
  * A post group entry must be a fluid node whose every wall link (0 <= q <= 1)
- * ends in a solid node: the kernel writes the re-entering populations into
- * elements only that node would touch, and reads the boundary node's own
- * post-collision elements back, while the launch is running.
+ * ends in a solid node.
  * Results equal vfx_k17_step + vfx_bc_apply bit for bit in every storage form. */
 vfx_status vfx_k17_step_fused(const vfx_lattice* lat, int32_t is_even_timestep, const vfx_fused_bc* post,
                               int32_t n_post, const vfx_fused_bc* pre, const uint32_t* any_mask, int32_t apply_pre,

@@ -1,0 +1,39 @@
+"""The pressure boundary inside the step on rows that are no multiple of a
+wavefront: boundary nodes fall on every lane, the first and the last among them
+(taken by the launch before the step).  The same bytes as the separate kernels,
+on both faces and in every storage form."""
+import numpy as np
+import pytest
+import torch
+
+import virtualfluids_amd as vfx
+from tests import cases
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("storage", ["fp64", "fp32", "fp16"])
+@pytest.mark.parametrize("normal", [1, 2])
+@pytest.mark.parametrize("nx", [5, 63, 64, 66, 70, 128, 130])
+def test_every_lane_gives_the_separate_kernels_bytes(cuda, nx, normal, storage):
+    print(f"[fused rows {nx} {normal} {storage}]", flush=True)
+    dims = (nx, 9, 8)
+    n = int(np.prod(dims))
+    solid = np.zeros(dims[::-1], bool)
+    solid[:, :, 0] = solid[:, :, -1] = True
+    yz = nx * np.arange(9 * 8)
+    nodes, inward = (yz + nx - 2, yz + nx - 3) if normal == 1 else (yz + 1, yz + 2)
+    rho = 1e-3 * np.cos(np.arange(nodes.size))
+    out = []
+    for fuse in (False, True):
+        lat = vfx.Lattice(dims, storage=storage, omega=1.9, solid=solid)
+        lat.init_equilibrium(*cases.random_flow(dims, seed=nx))
+        bc = vfx.BoundaryCondition(4, nodes, rho=rho, neighbors=inward, normal=normal)
+        st = vfx.Stepper(lat, "k17", [bc], fuse=fuse)
+        if fuse:  # the plan leaves entries with x mod 64 = 0 (63 for -x) to a kernel of their own
+            assert (st.fused_plan().pre is None) == (nx == 66 and normal == 1)
+        st.step(5)
+        st.step(2)
+        out.append(lat.f.view(torch.uint8))
+    assert torch.equal(*out)
+    assert n == lat.n_nodes

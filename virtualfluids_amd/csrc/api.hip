@@ -79,7 +79,6 @@ vfx_status make_lat(const vfx_lattice* in, vfx::Lat& L)
         L.nx = (uint32_t)nx;
         L.ny = (uint32_t)ny;
         L.nz = (uint32_t)nz;
-        L.chunks = (uint32_t)((nx + tile - 1) / tile);
         L.tile = in->tile_nodes;
         L.div_x = vfx::make_fastdiv(L.nx);
         L.div_y = vfx::make_fastdiv(L.ny);
@@ -557,14 +556,13 @@ vfx_status vfx_k17_step_fused(const vfx_lattice* lat, int32_t is_even, const vfx
     const double* lim = lat->quadric_limiter;
     switch (lat->storage) {
     case VFX_FP64:
-        e = vfx::launch_step_fused<double>(L, is_even != 0, lat->omega, lim, lat->force, g[0], g[1], g[2], any_mask, ap, st);
+        e = vfx::launch_step_fused<double>(L, is_even != 0, lat->omega, lim, lat->force, g[0], g[1], g[2], ap, st);
         break;
     case VFX_FP32:
-        e = vfx::launch_step_fused<float>(L, is_even != 0, lat->omega, lim, lat->force, g[0], g[1], g[2], any_mask, ap, st);
+        e = vfx::launch_step_fused<float>(L, is_even != 0, lat->omega, lim, lat->force, g[0], g[1], g[2], ap, st);
         break;
     default:
-        e = vfx::launch_step_fused<_Float16>(L, is_even != 0, lat->omega, lim, lat->force, g[0], g[1], g[2], any_mask, ap,
-                                             st);
+        e = vfx::launch_step_fused<_Float16>(L, is_even != 0, lat->omega, lim, lat->force, g[0], g[1], g[2], ap, st);
         break;
     }
     return hip_status(e, "fused collide-stream launch");

@@ -128,8 +128,8 @@ __device__ __forceinline__ uint32_t fastdiv(uint32_t n, const FastDiv& f)
 struct Lat {
     void* f;
     uint64_t N;
-    uint32_t nx, ny, nz, chunks; // direct addressing; chunks = blocks per x row (k_step_fused)
-    FastDiv div_x, div_y;        // division by nx, ny
+    uint32_t nx, ny, nz;  // direct addressing
+    FastDiv div_x, div_y; // division by nx, ny
     const uint32_t* solid;
     const uint32_t* nbx;
     const uint32_t* nby;
@@ -187,22 +187,6 @@ __host__ __device__ inline uint64_t node_items(const Lat& L, int direct)
 // The eight nodes a node's populations live on under the esoteric twist:
 // kk[b], bit0 = +x, bit1 = +y, bit2 = +z (VirtualFluids ListIndices,
 // KernelUtilities.h:221-245).
-__device__ __forceinline__ void nbrs_direct_xyz(const Lat& L, uint32_t x, uint32_t y, uint32_t z, uint32_t (&kk)[8])
-{
-    const uint32_t row = y + L.ny * z;
-    const uint32_t xp = (x + 1 == L.nx) ? 0u : x + 1;
-    const uint32_t ryp = (y + 1 == L.ny) ? row - y : row + 1;
-    const uint32_t rzp = (z + 1 == L.nz) ? y : row + L.ny;
-    const uint32_t ryzp = (y + 1 == L.ny) ? rzp - y : rzp + 1;
-    kk[0] = row * L.nx + x;
-    kk[1] = row * L.nx + xp;
-    kk[2] = ryp * L.nx + x;
-    kk[3] = ryp * L.nx + xp;
-    kk[4] = rzp * L.nx + x;
-    kk[5] = rzp * L.nx + xp;
-    kk[6] = ryzp * L.nx + x;
-    kk[7] = ryzp * L.nx + xp;
-}
 // interior node (no index wraps): one 24-bit multiply-add chain, then adds
 // of wave-uniform strides
 __device__ __forceinline__ void nbrs_interior(const Lat& L, uint32_t x, uint32_t y, uint32_t z, uint32_t (&kk)[8])
@@ -1327,24 +1311,6 @@ template <typename T> __device__ __forceinline__ void interp_wall_velocity(Inter
     }
 }
 
-// c_d . u with the direction's components given at run time (the order and
-// signs of proj())
-template <typename T> __device__ __forceinline__ T proj_rt(int ex, int ey, int ez, T ux, T uy, T uz)
-{
-    T v;
-    if (ex != 0) {
-        v = ex > 0 ? ux : -ux;
-        if (ey != 0) v = ey > 0 ? v + uy : v - uy;
-        if (ez != 0) v = ez > 0 ? v + uz : v - uz;
-    } else if (ey != 0) {
-        v = ey > 0 ? uy : -uy;
-        if (ez != 0) v = ez > 0 ? v + uz : v - uz;
-    } else {
-        v = ez > 0 ? uz : -uz;
-    }
-    return v;
-}
-
 // The population re-entering along a wall link of fraction q (0 <= q <= 1):
 // f, fi the node's post-collision populations of the link and its opposite,
 // w the link weight, vlb = c . u of the node, vbc = c . u of the wall.
@@ -1511,38 +1477,47 @@ template <typename T> __device__ __forceinline__ T feq_shifted(int d, T drho, T 
     return weight<T>(d) * (drho + (drho + T(1)) * (T(3) * cu + T(4.5) * cu * cu - cusq));
 }
 
-// PressureNonEquilibriumCompressible.cu: the inward neighbour's populations f
-// (by direction) with their equilibrium replaced by the one of the prescribed
-// density rho_bc, in place.
-template <typename T> __device__ __forceinline__ void pressure_values(T (&f)[27], T rho_bc)
+// PressureNonEquilibriumCompressible.cu: density deviation and velocity v of the
+// inward neighbour's populations (in cube order), and its population f of
+// direction d with the equilibrium replaced by the one of the prescribed density
+// rho_bc.  No FMA contraction: the same bits wherever they are inlined.
+template <typename T> __device__ __forceinline__ void pressure_moments(const T (&m)[27], T (&v)[4])
 {
-    // no FMA contraction: the same bits wherever the body is inlined
 #pragma clang fp contract(off)
+#define F(d) m[slot_of(d)]
     // getCompressibleMacroscopicValues (MacroscopicQuantities.h:117-127)
-    const T corners = ((f[dPPP] + f[dMMM]) + (f[dMPM] + f[dPMP])) + ((f[dMPP] + f[dPMM]) + (f[dMMP] + f[dPPM]));
-    const T edges = (((f[d0MP] + f[d0PM]) + (f[d0MM] + f[d0PP])) + ((f[dM0P] + f[dP0M]) + (f[dM0M] + f[dP0P]))) +
-                    ((f[dMP0] + f[dPM0]) + (f[dMM0] + f[dPP0]));
-    const T faces = ((f[dM00] + f[dP00]) + (f[d0M0] + f[d0P0])) + (f[d00M] + f[d00P]);
-    T drho1 = ((corners + edges) + f[d000]) + faces;
-    T vx1 = (((f[dPPP] - f[dMMM]) + (f[dPMP] - f[dMPM])) + ((f[dPMM] - f[dMPP]) + (f[dPPM] - f[dMMP]))) +
-            (((f[dP0M] - f[dM0P]) + (f[dP0P] - f[dM0M])) + ((f[dPM0] - f[dMP0]) + (f[dPP0] - f[dMM0]))) +
-            (f[dP00] - f[dM00]);
-    T vx2 = (((f[dPPP] - f[dMMM]) + (f[dMPM] - f[dPMP])) + ((f[dMPP] - f[dPMM]) + (f[dPPM] - f[dMMP]))) +
-            (((f[d0PM] - f[d0MP]) + (f[d0PP] - f[d0MM])) + ((f[dMP0] - f[dPM0]) + (f[dPP0] - f[dMM0]))) +
-            (f[d0P0] - f[d0M0]);
-    T vx3 = (((f[dPPP] - f[dMMM]) + (f[dPMP] - f[dMPM])) + ((f[dMPP] - f[dPMM]) + (f[dMMP] - f[dPPM]))) +
-            (((f[d0MP] - f[d0PM]) + (f[d0PP] - f[d0MM])) + ((f[dM0P] - f[dP0M]) + (f[dP0P] - f[dM0M]))) +
-            (f[d00P] - f[d00M]);
+    const T corners = ((F(dPPP) + F(dMMM)) + (F(dMPM) + F(dPMP))) + ((F(dMPP) + F(dPMM)) + (F(dMMP) + F(dPPM)));
+    const T edges = (((F(d0MP) + F(d0PM)) + (F(d0MM) + F(d0PP))) + ((F(dM0P) + F(dP0M)) + (F(dM0M) + F(dP0P)))) +
+                    ((F(dMP0) + F(dPM0)) + (F(dMM0) + F(dPP0)));
+    const T faces = ((F(dM00) + F(dP00)) + (F(d0M0) + F(d0P0))) + (F(d00M) + F(d00P));
+    const T drho1 = ((corners + edges) + F(d000)) + faces;
+    T vx1 = (((F(dPPP) - F(dMMM)) + (F(dPMP) - F(dMPM))) + ((F(dPMM) - F(dMPP)) + (F(dPPM) - F(dMMP)))) +
+            (((F(dP0M) - F(dM0P)) + (F(dP0P) - F(dM0M))) + ((F(dPM0) - F(dMP0)) + (F(dPP0) - F(dMM0)))) +
+            (F(dP00) - F(dM00));
+    T vx2 = (((F(dPPP) - F(dMMM)) + (F(dMPM) - F(dPMP))) + ((F(dMPP) - F(dPMM)) + (F(dPPM) - F(dMMP)))) +
+            (((F(d0PM) - F(d0MP)) + (F(d0PP) - F(d0MM))) + ((F(dMP0) - F(dPM0)) + (F(dPP0) - F(dMM0)))) +
+            (F(d0P0) - F(d0M0));
+    T vx3 = (((F(dPPP) - F(dMMM)) + (F(dPMP) - F(dMPM))) + ((F(dMPP) - F(dPMM)) + (F(dMMP) - F(dPPM)))) +
+            (((F(d0MP) - F(d0PM)) + (F(d0PP) - F(d0MM))) + ((F(dM0P) - F(dP0M)) + (F(dP0P) - F(dM0M)))) +
+            (F(d00P) - F(d00M));
     const T oor = T(1) / (drho1 + T(1));
-    vx1 *= oor;
-    vx2 *= oor;
-    vx3 *= oor;
-    const T cusq = T(1.5) * (vx1 * vx1 + vx2 * vx2 + vx3 * vx3);
-#pragma unroll
-    for (int d = 0; d < 27; ++d) f[d] -= feq_shifted<T>(d, drho1, vx1, vx2, vx3, cusq);
-    drho1 = rho_bc;
-#pragma unroll
-    for (int d = 0; d < 27; ++d) f[d] += feq_shifted<T>(d, drho1, vx1, vx2, vx3, cusq);
+#undef F
+    v[0] = drho1;
+    v[1] = vx1 * oor;
+    v[2] = vx2 * oor;
+    v[3] = vx3 * oor;
+}
+template <typename T> __device__ __forceinline__ T pressure_value(int d, T f, const T (&v)[4], T rho_bc)
+{
+#pragma clang fp contract(off)
+    const T cusq = T(1.5) * (v[1] * v[1] + v[2] * v[2] + v[3] * v[3]);
+    if constexpr (sizeof(T) == 4) {
+        // the two equilibria differ by w (rho_bc - drho) (1 + 3 cu + 4.5 cu^2 - cusq)
+        const T cu = d == d000 ? T(0) : proj<T>(d, v[1], v[2], v[3]);
+        const T e = __builtin_fmaf(__builtin_fmaf(T(4.5), cu, T(3)), cu, T(1) - cusq);
+        return __builtin_fmaf(weight<T>(d) * (rho_bc - v[0]), e, f);
+    }
+    return (f - feq_shifted<T>(d, v[0], v[1], v[2], v[3], cusq)) + feq_shifted<T>(d, rho_bc, v[1], v[2], v[3], cusq);
 }
 
 template <typename S, bool EVEN>
@@ -1562,15 +1537,15 @@ __device__ __forceinline__ void bc_pressure_entry(const Lat& L, const BCDev& B, 
     }
     T m[27];
     gather<S, T, EVEN>(L, kkn, m);
-    T f[27];
-#pragma unroll
-    for (int s = 0; s < 27; ++s) f[dir_at(s)] = m[s];
-    pressure_values<T>(f, bc_at<T>(B.rho, i));
+    T v[4];
+    pressure_moments<T>(m, v);
+    const T rho_bc = bc_at<T>(B.rho, i);
     const int nx = cx(B.normal), ny = cy(B.normal), nz = cz(B.normal);
 #pragma unroll
     for (int d = 0; d < 27; ++d) {
         if (cx(d) * nx + cy(d) * ny + cz(d) * nz > 0) continue;
-        Storage<S, T>::st(plane<S>(L, slot(d, EVEN)), kk[nbr(d)], f[d], L.st[weight_class(d)], L.ss[d]);
+        Storage<S, T>::st(plane<S>(L, slot(d, EVEN)), kk[nbr(d)], pressure_value<T>(d, m[slot_of(d)], v, rho_bc),
+                          L.st[weight_class(d)], L.ss[d]);
     }
 }
 
@@ -1578,6 +1553,14 @@ template <typename S, bool EVEN>
 __global__ void __launch_bounds__(256) k_bc_pressure(Lat L, BCDev B)
 {
     bc_pressure_entry<S, EVEN>(L, B, blockIdx.x * blockDim.x + threadIdx.x);
+}
+// the entries k_step_pre leaves out: nodes in the wavefront's first lane (last,
+// for an outward normal -x)
+template <typename S, bool EVEN>
+__global__ void __launch_bounds__(256) k_bc_pressure_edge(Lat L, BCDev B)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < B.n && (B.k[i] & 63u) == (B.normal == dP00 ? 0u : 63u)) bc_pressure_entry<S, EVEN>(L, B, i);
 }
 
 // Several boundary groups, possibly of different lattices of one storage
@@ -1854,25 +1837,17 @@ __global__ void __launch_bounds__(256) k_bc_outflow(Lat L, BCDev B)
 }
 
 // ---------------------------------------------- fused boundary conditions ----
-// Boundary conditions applied inside the collide-stream kernel of a structured
-// (direct) lattice, so that a boundary node's 27 populations are not read a
-// second time by a kernel of its own.  On a face normal to x every element a
-// boundary node touches sits in its own cache line (x is the fastest index),
-// so a separate boundary kernel moves ~64 times the bytes it uses.
-//  * post-collision interpolated kinds (1 no-slip, 2 velocity, 3 slip, 5
-//    velocity with pressure): the thread that collided node k computes the
-//    re-entering populations from its post-collision values and stores them,
-//    as k_bc_interp would right after the kernel (the element written belongs
-//    to the wall node, which no thread of the launch touches);
-//  * the non-equilibrium pressure boundary on a face normal to +-x
-//    (PressureNonEquilibriumCompressible, pre-collision): node k's incoming
-//    populations are replaced at the start of the next step from its inward
-//    neighbour k -+ 1, whose pre-collision populations the neighbouring lane
-//    of the same wavefront has just gathered (cross-lane shuffle), instead of
-//    by a kernel after the parity flip.  The values are the ones that kernel
-//    would store and the collision read back (the storage round trip is
-//    applied), so fused and separate runs agree bit for bit.
-// Node k belongs to a group iff bit k of `mask` is set; its entry is
+// The non-equilibrium pressure boundary on a face normal to +-x
+// (PressureNonEquilibriumCompressible, pre-collision) inside the collide-stream
+// kernel of a structured (direct) lattice: on such a face every element a
+// boundary node touches sits in its own cache line (x is the fastest index), so
+// a boundary kernel moves ~64 times the bytes it uses.  Node k's incoming
+// populations are replaced at the start of the next step from its inward
+// neighbour k -+ 1, whose pre-collision populations the lane beside it has just
+// gathered, instead of by a kernel after the parity flip.  The values are the
+// ones that kernel would store and the collision read back (the storage round
+// trip is applied), so fused and separate runs agree bit for bit.
+// Node k belongs to the group iff bit k of `mask` is set; its entry is
 // base[k/32] + the number of set bits below it in its word (entries sorted by
 // node).
 struct FusedGroup {
@@ -1882,20 +1857,6 @@ struct FusedGroup {
     int32_t kind;
 };
 
-__device__ __forceinline__ bool in_group(const FusedGroup& G, uint32_t k)
-{
-    return G.mask && ((G.mask[k >> 5] >> (k & 31u)) & 1u);
-}
-
-__device__ __forceinline__ bool fused_entry(const FusedGroup& G, uint32_t k, uint32_t& i)
-{
-    const uint32_t w = G.mask[k >> 5];
-    const uint32_t b = k & 31u;
-    if (!((w >> b) & 1u)) return false;
-    i = G.base[k >> 5] + (uint32_t)__builtin_popcount(w & ((1u << b) - 1u));
-    return i < G.B.n && G.B.k[i] == k; // malformed tables select nothing
-}
-
 // what a store of v as direction d followed by a load gives back (the value
 // the separate boundary kernels exchange through memory)
 template <typename S, typename T> __device__ __forceinline__ T round_trip(T v, float st, float ss, float ld, float sh)
@@ -1904,216 +1865,89 @@ template <typename S, typename T> __device__ __forceinline__ T round_trip(T v, f
     else return v;
 }
 
-template <typename S, typename T, bool EVEN>
-__device__ __forceinline__ void fused_post(const Lat& L, const FusedGroup& G, uint32_t k)
+// x of the lane before this one (PX) or after it, across the whole wavefront
+// (DPP wave_shr / wave_shl; the end lane, which has no such lane, gets 0)
+template <bool PX> __device__ __forceinline__ float lane_beside(float x)
 {
-    uint32_t i;
-    if (!fused_entry(G, k, i)) return;
-    // The neighbour indices are recomputed from an index opaque to the
-    // compiler: otherwise it keeps them, or the 64-bit element addresses of
-    // the scatter, for the loads below and spills them on every node.
-    asm volatile("" : "+v"(k));
-    uint32_t kb[8];
-    nbrs_direct(L, k, kb);
-    // the node's post-collision populations, read back from the elements this
-    // thread has just stored them to (no other node writes those elements in
-    // the step): keeping the 27 collision outputs in registers for this rarely
-    // taken path would spill them on every node
-    T p[27];
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), PX ? 0x138 : 0x130, 0xf, 0xf, true));
+}
+template <bool PX> __device__ __forceinline__ double lane_beside(double x)
+{
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    const uint64_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, PX ? 0x138 : 0x130, 0xf, 0xf, true);
+    const uint64_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), PX ? 0x138 : 0x130, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, hi << 32 | lo);
+}
+// the boundary nodes of a wavefront take their values from the lane beside them
+// (PX: outward normal +x, the inward neighbour is the lane before); every lane
+// of the wavefront runs this
+template <typename S, typename T, bool PX>
+__device__ __forceinline__ void fused_pressure(const Lat& L, const FusedGroup& G, bool mine, T rho_bc, T (&m)[27])
+{
+    T own[4], v[4];
+    pressure_moments<T>(m, own);
 #pragma unroll
-    for (int d = 0; d < 27; ++d) {
-        const int e = inv(d);
-        p[d] = Storage<S, T>::ld(plane<S>(L, slot(e, EVEN)), kb[nbr(e)], L.ld[weight_class(d)], L.sh[d]);
+    for (int c = 0; c < 4; ++c) v[c] = lane_beside<PX>(own[c]);
+#pragma unroll
+    for (int s = 0; s < 27; ++s) {
+        const int d = dir_at(s);
+        if (PX ? cx(d) > 0 : cx(d) < 0) continue; // pointing out of the domain
+        const int c = weight_class(d);
+        const T f = round_trip<S, T>(pressure_value<T>(d, lane_beside<PX>(m[s]), v, rho_bc), L.st[c], L.ss[d], L.ld[c], L.sh[d]);
+        m[s] = mine ? f : m[s];
     }
-    interp_links<S, T, EVEN, -1>(L, G.B, i, kb[0], kb, p, G.kind);
 }
 
-// Link-parallel form of fused_post for a wavefront with few boundary nodes:
-// the wavefront takes its boundary nodes one after another, lane x (< 27)
-// loads the node's post-collision population of direction x, the lanes share
-// them, and lane d (1..26) computes and stores the re-entering population of
-// link d.  The node part and every link value are the expressions of
-// interp_links (kinds 1, 2, 5; slip marks its face axes in link order and
-// stays per node), so the results are the same bits.
-constexpr uint32_t kLinkParallelNodes = 8; // boundary nodes per wavefront up to which links go across lanes
-struct LaneDir {
-    int x;              // direction of this lane (0 for lanes >= 27)
-    int ix;             // the opposite direction
-    int ex, ey, ez;     // components of x
-    uint32_t rd_plane;  // plane of the node's post-collision population x
-    uint32_t wr_plane;  // plane of the re-entering population of link x
-    uint32_t nbsel;     // which of the node's 8 neighbour indices holds both
-    float ld, sh, st, ss;
-};
-template <bool EVEN> __device__ __forceinline__ LaneDir lane_dir(const Lat& L, int lane)
-{
-    LaneDir r;
-    const int x = lane < 27 ? lane : 0;
-    r.x = x;
-    int ex = 0, ey = 0, ez = 0, ix = 0;
-    float sh = 0.f, ss = 0.f;
-    // constant-index selects: the kernel argument arrays stay in place
-#pragma unroll
-    for (int d = 0; d < 27; ++d) {
-        if (x == d) {
-            ex = cx(d);
-            ey = cy(d);
-            ez = cz(d);
-            ix = inv(d);
-            sh = L.sh[d];
-            ss = L.ss[inv(d)];
-        }
-    }
-    r.ix = ix;
-    r.ex = ex;
-    r.ey = ey;
-    r.ez = ez;
-    // population x is read where direction inv(x) is read (slot(inv(x), EVEN));
-    // link x re-enters as inv(x), written at slot(inv(x), !EVEN); both at the
-    // neighbour that is one step along every axis where c_x > 0
-    r.rd_plane = (uint32_t)(EVEN ? ix : x);
-    r.wr_plane = (uint32_t)(EVEN ? x : ix);
-    r.nbsel = (uint32_t)((ex > 0) | ((ey > 0) << 1) | ((ez > 0) << 2));
-    const int c = (ex != 0) + (ey != 0) + (ez != 0);
-    r.ld = c == 0 ? L.ld[0] : c == 1 ? L.ld[1] : c == 2 ? L.ld[2] : L.ld[3];
-    r.st = c == 0 ? L.st[0] : c == 1 ? L.st[1] : c == 2 ? L.st[2] : L.st[3];
-    r.sh = sh;
-    r.ss = ss;
-    return r;
-}
-template <typename T> __device__ __forceinline__ T weight_rt(int ex, int ey, int ez)
-{
-    const int c = (ex != 0) + (ey != 0) + (ez != 0);
-    return c == 0 ? T(8. / 27.) : c == 1 ? T(2. / 27.) : c == 2 ? T(1. / 54.) : T(1. / 216.);
-}
-template <typename S, typename T, bool EVEN>
-__device__ __forceinline__ void fused_post_links(const Lat& L, const FusedGroup& G, uint32_t kb, int lane,
-                                                 const LaneDir& D)
-{
-    uint32_t i;
-    if (!fused_entry(G, kb, i)) return; // the same for every lane
-    uint32_t nb[8];
-    nbrs_direct(L, kb, nb);
-    uint32_t idx = nb[0];
-#pragma unroll
-    for (int j = 1; j < 8; ++j)
-        if (D.nbsel == (uint32_t)j) idx = nb[j];
-    const T px = Storage<S, T>::ld(plane<S>(L, (int)D.rd_plane), idx, D.ld, D.sh);
-    T p[27];
-#pragma unroll
-    for (int d = 0; d < 27; ++d) p[d] = __shfl(px, d, 64);
-    const int kd = G.kind;
-    InterpNode<T> n = interp_node<T, -1>(L, G.B, i, kb, p, kd);
-    T q = T(-1);
-    if (lane >= 1 && lane < 27) q = bc_q<T>(G.B, lane, i);
-    interp_wall_velocity<T>(n, G.B, i, kd);
-    const T fi = __shfl(px, D.ix, 64);
-    if (!(lane >= 1 && lane < 27) || !(q >= T(0) && q <= T(1))) return;
-    const T w = weight_rt<T>(D.ex, D.ey, D.ez);
-    const T vlb = proj_rt<T>(D.ex, D.ey, D.ez, n.vx1, n.vx2, n.vx3);
-    const T vbc = kd == VFX_BC_NOSLIP_INTERPOLATED ? T(0) : proj_rt<T>(D.ex, D.ey, D.ez, n.VX, n.VY, n.VZ);
-    const T v = interp_link_value<T>(n, kd, w, vlb, vbc, q, px, fi);
-    Storage<S, T>::st(plane<S>(L, (int)D.wr_plane), idx, v, D.st, D.ss);
-}
-
-// K17 (default operation order of the storage form) with up to two fused
-// post-collision groups and one fused pressure group; apply_pre = 0 on the
-// first step of a run (no pressure boundary ran before it).
-// The boundary paths need more registers than the collision; the occupancy of
-// the plain kernel (7 waves per SIMD at <= 72 VGPRs for 2- and 4-byte storage)
-// is kept by capping the register budget, so that those rarely taken paths
-// spill instead.
-template <typename S> constexpr int fused_waves() { return sizeof(S) == 8 ? 3 : 7; }
+// The structured K17 step with the pressure group inside: where a wavefront
+// holds boundary nodes, each takes its neighbour's populations from the lane
+// beside it.  It costs its instructions (~250) and one more round trip to memory
+// in the wavefronts that hold a boundary node, where a kernel of its own reads
+// 27 and writes 18 cache lines per node of the face.  Every lane forms its own
+// density and velocity and the lanes pass one population at a time, so no second
+// set of 27 registers is live (73 VGPRs for FP16, nothing spilled; held to 72
+// the step schedules worse, 190 us); the group's words are read before the
+// populations, the entry while they arrive (after them: 150 us).  A boundary
+// node whose neighbour is in another wavefront (lane 0, or 63 for -x) is left to
+// k_bc_pressure_edge, launched before.  MI355X, FP16 channel 288x144x144: 135 us
+// + 4.6 for the edge, against 123 + 32 for the plain step and k_bc_pressure.
 template <typename S, bool EVEN>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves<S>())))
-    k_step_fused(Lat L, Rates<typename Compute<S>::T> R, FusedGroup g0, FusedGroup g1, FusedGroup gp,
-                 const uint32_t* any, int32_t apply_pre)
+__global__ void __launch_bounds__(256) k_step_pre(Lat L, Rates<typename Compute<S>::T> R, FusedGroup gp)
 {
     using T = typename Compute<S>::T;
     constexpr bool FAST = sizeof(S) != 8;
     constexpr bool O2 = sizeof(S) == 2;
-    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x, xcd_run<S>());
-    const uint32_t row = blk / L.chunks;
-    const uint32_t x = (blk - row * L.chunks) * blockDim.x + threadIdx.x;
-    const uint32_t y = row % L.ny, z = row / L.ny;
+    const uint32_t blk = L.xrun_lg ? xcd_block_pow2(blockIdx.x, gridDim.x, L.xrun_lg - 1u)
+                                   : xcd_block(blockIdx.x, gridDim.x, step_run<S>());
+    const uint32_t k = blk * blockDim.x + threadIdx.x;
+    const bool active = k < (uint32_t)L.N && !is_solid(L, k);
+    // the group's words are read before the populations, so that a boundary
+    // node's entry is on its way while they arrive
+    const uint32_t at = active ? k >> 5 : 0u, word = gp.mask[at], base = gp.base[at];
     uint32_t kk[8];
-    nbrs_direct_xyz(L, x < L.nx ? x : L.nx - 1, y, z, kk);
-    const bool active = x < L.nx && !is_solid(L, kk[0]);
-    // union of the groups' node masks, loaded with the populations: nodes of
-    // no group (most of them) take no further round trip to memory
-    const bool member = any == nullptr || ((any[kk[0] >> 5] >> (kk[0] & 31u)) & 1u);
+    nbrs_direct(L, k, kk);
     T m[27], mv[4], nut = T(0);
 #pragma unroll
     for (int s = 0; s < 27; ++s) m[s] = T(0);
     if (active) gather<S, T, EVEN>(L, kk, m);
-    if (gp.mask && apply_pre && __ballot(active && member)) {
-        uint32_t ip = 0;
-        const bool pl = active && member && fused_entry(gp, kk[0], ip);
-        if (__ballot(pl)) {
-            // inward neighbour k - 1 (outward normal +x) or k + 1 (-x): the lane next to this one
-            const int lane = (int)(threadIdx.x & 63u);
-            const int src = gp.B.normal == dP00 ? lane - 1 : lane + 1;
-            T f[27];
-#pragma unroll
-            for (int s = 0; s < 27; ++s) f[dir_at(s)] = __shfl(m[s], src & 63, 64);
-            const uint32_t kn = gp.B.normal == dP00 ? kk[0] - 1u : kk[0] + 1u;
-            const bool row = gp.B.normal == dP00 ? x >= 1u : x + 1u < L.nx; // neighbour in this row
-            if (pl && row && src >= 0 && src < 64 && gp.B.kn[ip] == kn) {
-                pressure_values<T>(f, bc_at<T>(gp.B.rho, ip));
-                const int ncx = cx(gp.B.normal);
-#pragma unroll
-                for (int s = 0; s < 27; ++s) {
-                    const int d = dir_at(s);
-                    if (cx(d) * ncx > 0) continue;
-                    const int c = weight_class(d);
-                    m[s] = round_trip<S, T>(f[d], L.st[c], L.ss[d], L.ld[c], L.sh[d]);
-                }
-            }
+    const bool px = gp.B.normal == dP00; // outward normal +x: the inward neighbour is the lane before
+    const bool member = active && ((word >> (k & 31u)) & 1u);
+    if (__ballot(member)) {
+        const uint32_t i = base + (uint32_t)__builtin_popcount(word & ((1u << (k & 31u)) - 1u));
+        bool mine = member && i < gp.B.n && (threadIdx.x & 63u) != (px ? 0u : 63u);
+        uint32_t ek = 0, ekn = 0;
+        T rho_bc = T(0);
+        if (mine) {
+            ek = gp.B.k[i];
+            ekn = gp.B.kn[i];
+            rho_bc = bc_at<T>(gp.B.rho, i);
         }
+        mine = mine && ek == k && ekn == (px ? k - 1u : k + 1u); // malformed tables select nothing
+        if (px) fused_pressure<S, T, true>(L, gp, mine, rho_bc, m);
+        else fused_pressure<S, T, false>(L, gp, mine, rho_bc, m);
     }
-    // lanes without a node stay for the link-parallel boundary path below
-    if (active) {
-        collide<T, VFX_K17, FAST, O2>(m, R, mv, nut);
-        scatter_post<S, T, EVEN, O2>(L, kk, m);
-    }
-    // the boundary code reads the stores above back from memory
-    asm volatile("" ::: "memory");
-    // only wavefronts with nodes of a group go on (whatever the boundary code
-    // needs is set up behind this branch, not on every node)
-    const uint32_t k = kk[0];
-    const bool bc = active && member && (in_group(g0, k) || in_group(g1, k));
-    const uint64_t any_bc = __ballot(bc);
-    if (!any_bc) return;
-    const int lane = (int)(threadIdx.x & 63u);
-    if (__popcll(any_bc) <= kLinkParallelNodes) {
-        // the stores of other lanes are read back
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-        const LaneDir D = lane_dir<EVEN>(L, lane);
-#pragma unroll 1
-        for (int j = 0; j < 2; ++j) {
-            const FusedGroup& G = j == 0 ? g0 : g1;
-            if (!G.mask) continue;
-            const bool mine = bc && in_group(G, k);
-            uint64_t bal = __ballot(mine);
-            if (G.kind == VFX_BC_SLIP) {
-                if (mine) fused_post<S, T, EVEN>(L, G, k);
-                continue;
-            }
-            while (bal) {
-                const int b = __builtin_ctzll(bal);
-                bal &= bal - 1;
-                fused_post_links<S, T, EVEN>(L, G, (uint32_t)__shfl((int)k, b, 64), lane, D);
-            }
-        }
-        return;
-    }
-    if (!bc) return;
-    // one inlined copy of the boundary code serves both groups
-#pragma unroll 1
-    for (int j = 0; j < 2; ++j) {
-        const FusedGroup& G = j == 0 ? g0 : g1;
-        if (G.mask) fused_post<S, T, EVEN>(L, G, k);
-    }
+    if (!active) return;
+    collide<T, VFX_K17, FAST, O2>(m, R, mv, nut);
+    scatter_post<S, T, EVEN, O2>(L, kk, m);
 }
 
 // The coarse step and the first fine step of a nest (or any two structured
@@ -2493,21 +2327,42 @@ template <typename S> hipError_t launch_step(const Lat& L, int direct, int coll,
     return launch_step_p<S, VFX_BGK>(L, direct, even, false, R, st);
 }
 
-// K17 collide-and-stream of a structured lattice with fused boundary groups
-// (k_step_fused); same grid as the direct k_step_direct launch
+template <typename S> hipError_t launch_bc(const Lat& L, const BCDev& B, int kind, bool even, hipStream_t st);
+
+// K17 collide-and-stream of a structured lattice with its boundary groups: the
+// pressure group inside the step (k_step_pre), the post-collision ones after it
+// by their own kernels.  Inside the step a post-collision boundary node costs
+// its whole wavefront the boundary code and several dependent round trips: every
+// group of the 512x256x256 channel inside 1195 us against 1003 apart, the inlet
+// alone +140 against +94 (FP16, MI355X).
 template <typename S>
 hipError_t launch_step_fused(const Lat& L, bool even, double omega, const double* lim, const double* force,
-                             const FusedGroup& g0, const FusedGroup& g1, const FusedGroup& gp, const uint32_t* any,
-                             int apply_pre, hipStream_t st)
+                             const FusedGroup& g0, const FusedGroup& g1, const FusedGroup& gp, int apply_pre,
+                             hipStream_t st)
 {
     using T = typename Compute<S>::T;
     const Rates<T> R = make_rates<T>(omega, lim, force, 0.0);
-    const unsigned grid = L.chunks * L.ny * L.nz;
-    const unsigned block = (unsigned)((L.nx + L.chunks - 1) / L.chunks);
-    const unsigned b = block <= 64 ? 64 : block <= 128 ? 128 : 256;
-    if (even) hipLaunchKernelGGL((k_step_fused<S, true>), dim3(grid), dim3(b), 0, st, L, R, g0, g1, gp, any, apply_pre);
-    else hipLaunchKernelGGL((k_step_fused<S, false>), dim3(grid), dim3(b), 0, st, L, R, g0, g1, gp, any, apply_pre);
-    return hipGetLastError();
+    hipError_t e = hipSuccess;
+    if (gp.mask && apply_pre) {
+        const dim3 edge(grid_for(gp.B.n, kBlock)), b(kBlock);
+        // rows of whole wavefronts keep the pair in one (the caller's x mod 64 condition)
+        if (L.nx % 64u != 0) {
+            if (even) hipLaunchKernelGGL((k_bc_pressure_edge<S, true>), edge, b, 0, st, L, gp.B);
+            else hipLaunchKernelGGL((k_bc_pressure_edge<S, false>), edge, b, 0, st, L, gp.B);
+        }
+        const unsigned tile = L.tile ? L.tile : sizeof(S) == 4 ? 128u : 256u;
+        const dim3 g(grid_for(L.N, tile)), t(tile);
+        constexpr unsigned lds = step_lds_cap<S, VFX_K17, sizeof(S) != 8>();
+        if (even) hipLaunchKernelGGL((k_step_pre<S, true>), g, t, lds, st, L, R, gp);
+        else hipLaunchKernelGGL((k_step_pre<S, false>), g, t, lds, st, L, R, gp);
+        e = hipGetLastError();
+    } else {
+        constexpr bool FAST = sizeof(S) != 8;
+        e = even ? launch_step_t<S, VFX_K17, true, FAST>(L, 1, R, st) : launch_step_t<S, VFX_K17, false, FAST>(L, 1, R, st);
+    }
+    if (e == hipSuccess && g0.mask) e = launch_bc<S>(L, g0.B, g0.kind, even, st);
+    if (e == hipSuccess && g1.mask) e = launch_bc<S>(L, g1.B, g1.kind, even, st);
+    return e;
 }
 
 template <typename S>
@@ -2801,7 +2656,7 @@ template <typename S> hipError_t launch_bc(const Lat& L, const BCDev& B, int kin
     template hipError_t launch_step<S>(const Lat&, int, int, bool, int, double, const double*, const double*, int,      \
                                        double, hipStream_t);                                                           \
     template hipError_t launch_step_fused<S>(const Lat&, bool, double, const double*, const double*, const FusedGroup&, \
-                                             const FusedGroup&, const FusedGroup&, const uint32_t*, int, hipStream_t); \
+                                             const FusedGroup&, const FusedGroup&, int, hipStream_t); \
     template hipError_t launch_turb_amd<S>(const Lat&, int, double, hipStream_t);                                      \
     template hipError_t launch_bc_set<S>(const BCJob*, uint32_t, uint32_t, uint32_t, hipStream_t);                    \
     template hipError_t launch_step_levels<S>(const LevelInput*, int, hipStream_t);                                    \
@@ -2827,7 +2682,7 @@ template <typename S> hipError_t launch_bc(const Lat& L, const BCDev& B, int kin
                                               int, double, hipStream_t);                                               \
     extern template hipError_t launch_step_fused<S>(const Lat&, bool, double, const double*, const double*,            \
                                                     const FusedGroup&, const FusedGroup&, const FusedGroup&,           \
-                                                    const uint32_t*, int, hipStream_t);                                \
+                                                    int, hipStream_t);                                                 \
     extern template hipError_t launch_turb_amd<S>(const Lat&, int, double, hipStream_t);                               \
     extern template hipError_t launch_bc_set<S>(const BCJob*, uint32_t, uint32_t, uint32_t, hipStream_t);             \
     extern template hipError_t launch_step_levels<S>(const LevelInput*, int, hipStream_t);                             \

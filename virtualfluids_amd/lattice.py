@@ -300,7 +300,7 @@ class Lattice:
         V.check(V.lib().vfx_bc_apply(C.byref(s), C.byref(b), int(bool(even)), _stream(stream)), "vfx_bc_apply")
 
     def k17_step_fused(self, even, post=(), pre=None, apply_pre=False, any_mask=None, stream=None):
-        """K17 collide+stream with boundary groups applied inside the kernel
+        """K17 collide+stream with its boundary groups in one call
         (vfx_k17_step_fused): up to two post-collision FusedGroups and one
         pressure FusedGroup whose values the step takes from the previous
         step's populations (apply_pre False on the first step of a run);
@@ -864,8 +864,8 @@ def step_levels(levels, stream=None):
 
 @dataclass
 class FusedPlan:
-    """Which boundary entries a fused step applies inside the collide-stream
-    kernel (post: up to two groups, pre: one pressure group) and which run as
+    """Which boundary entries a fused step takes along (post: up to two groups,
+    pre: one pressure group, inside the collide-stream kernel) and which run as
     boundary kernels of their own (residual_post / residual_pre, in the order
     of the unfused step)."""
 
@@ -943,10 +943,8 @@ class Stepper:
     # kernel where the geometry allows (FusedPlan); same populations as the
     # separate boundary kernels.
     fuse: bool = False
-    # with fuse: also the interpolated kinds (False: the pressure group only).
-    # Inside the kernel a boundary node costs its whole wavefront the boundary
-    # code; on a face normal to x that is one node in 64, where a separate
-    # kernel runs 64 boundary nodes per wavefront.
+    # with fuse: also the interpolated kinds are part of the step's call (False:
+    # the pressure group only); they run as kernels of their own either way
     fuse_post: bool = True
     # Before the first step, apply the non-reflecting outflow kinds once with
     # the starting parity: they write the populations the step after next

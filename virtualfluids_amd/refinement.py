@@ -471,7 +471,8 @@ class RefinedStepper:
         """Kernel launches of one coarse step in the current schedule."""
         if self._plan_c is not None:
             p = self._plan_c
-            return 2 * (1 + len(self.fine_bcs)) + 1 + len(p.residual_post) + len(p.residual_pre) + 2
+            edge = int(self.coarse.dims[0] % 64 != 0)  # outlet nodes whose neighbour is in another wavefront
+            return 2 * (1 + len(self.fine_bcs)) + 1 + edge + len(p.residual_post) + len(p.residual_pre) + 2
         if self.merged:
             sets = (self._set_post_both, self._set_pre_both, self._set_post_fine, self._set_pre_fine)
             rest = 2 * (len(self._f_post_rest) + len(self._f_pre_rest)) + len(self._c_post_rest) + len(self._c_pre_rest)
