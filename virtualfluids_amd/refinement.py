@@ -244,19 +244,27 @@ def scale_fc_cf(coarse: Lattice, fine: Lattice, fc: ICells, cf: ICells, coarse_e
                                     int(bool(fine_even)), _stream(stream)), "vfx_scale_fc_cf")
 
 
-def _cell_corners(base, dims):
+def _corners(base, dims):
     """The 8 corner nodes (x fastest, periodic wrap) of the cells at `base`
-    of a structured box, as the interface kernels take them."""
+    of a structured box, as the interface kernels take them, one array per corner."""
     nx, ny, nz = dims
-    base = np.asarray(base, dtype=np.int64)
-    x, y, z = base % nx, (base // nx) % ny, base // (nx * ny)
-    out = []
+    base = np.asarray(base).astype(np.int32 if nx * ny * nz < 2 ** 31 else np.int64)
+    r = base // nx
+    z = r // ny
+    dx = np.where(base - r * nx + 1 == nx, 1 - nx, 1).astype(base.dtype)
+    dy = np.where(r - z * ny + 1 == ny, nx - nx * ny, nx).astype(base.dtype)
+    dz = np.where(z + 1 == nz, nx * ny * (1 - nz), nx * ny).astype(base.dtype)
     for c in range(8):
-        xx = (x + (c & 1)) % nx
-        yy = (y + ((c >> 1) & 1)) % ny
-        zz = (z + ((c >> 2) & 1)) % nz
-        out.append(xx + nx * (yy + ny * zz))
-    return np.concatenate(out) if base.size else np.zeros(0, np.int64)
+        k = base
+        for bit, step in ((1, dx), (2, dy), (4, dz)):
+            if c & bit:
+                k = k + step
+        yield k
+
+
+def _cell_corners(base, dims):
+    """_corners as one array, corner by corner."""
+    return np.concatenate([np.asarray(k, dtype=np.int64) for k in _corners(base, dims)])
 
 
 def interface_cells_apart(nest) -> bool:
@@ -264,11 +272,17 @@ def interface_cells_apart(nest) -> bool:
     node the fine-to-coarse cells write is a corner of a coarse-to-fine cell,
     and no fine node the coarse-to-fine cells write is a corner of a
     fine-to-coarse cell."""
-    fc_targets = np.asarray(nest.fc_coarse, dtype=np.int64)
-    cf_sources = _cell_corners(nest.cf_coarse, nest.coarse_dims)
-    fc_sources = _cell_corners(nest.fc_fine, nest.fine_dims)
-    cf_targets = _cell_corners(nest.cf_fine, nest.fine_dims)
-    return not (np.intersect1d(fc_targets, cf_sources).size or np.intersect1d(fc_sources, cf_targets).size)
+    def marked(nodes, dims):
+        m = np.zeros(int(np.prod(dims)), dtype=bool)
+        for k in nodes:
+            m[k] = True
+        return m
+
+    coarse = marked([np.asarray(nest.fc_coarse)], nest.coarse_dims)
+    if any(coarse[k].any() for k in _corners(nest.cf_coarse, nest.coarse_dims)):
+        return False
+    fine = marked(_corners(nest.cf_fine, nest.fine_dims), nest.fine_dims)
+    return not any(fine[k].any() for k in _corners(nest.fc_fine, nest.fine_dims))
 
 
 def fine_omega(omega_coarse: float) -> float:
@@ -318,6 +332,10 @@ class RefinedStepper:
             bc.tables(real)
         self.fc.offsets(real)
         self.cf.offsets(real)
+        # both interface interpolations in one launch where the nest keeps them
+        # apart: each alone is bound by latency and by the cache lines of the
+        # faces normal to x
+        self._one_interface = interface_cells_apart(nest)
         self.merged = bool(merged)
         if self.merged:
             self._setup_merged()
@@ -359,7 +377,6 @@ class RefinedStepper:
         self._set_pre_both = BCSet([(self.coarse, b) for b in cpre] + [(self.fine, b) for b in fpre])
         self._set_pre_fine = BCSet([(self.fine, b) for b in fpre])
         self._n_fpost, self._n_fpre = len(fpost), len(fpre)
-        self._one_interface = interface_cells_apart(self.nest)
 
     def _step_merged(self, stream):
         c, f = self.coarse, self.fine
@@ -387,6 +404,10 @@ class RefinedStepper:
         for b in self._f_pre_rest:
             f.apply_bc(b, ef, stream=stream)
         self.even_c, self.even_f = ec, ef
+        self._interface(stream)
+
+    def _interface(self, stream):
+        c, f, ec, ef = self.coarse, self.fine, self.even_c, self.even_f
         if self._one_interface:
             scale_fc_cf(c, f, self.fc, self.cf, ec, ef, stream)
         else:
@@ -427,8 +448,7 @@ class RefinedStepper:
                 self.even_c = self._coarse_step_fused(self.even_c, i == 0, stream)
             else:
                 self.even_c = self._level_step(self.coarse, self.coarse_bcs, self.collision, self.even_c, stream)
-            scale_fc(self.coarse, self.fine, self.fc, self.even_c, self.even_f, stream)
-            scale_cf(self.coarse, self.fine, self.cf, self.even_c, self.even_f, stream)
+            self._interface(stream)
         if n > 0 and self._plan_c is not None:
             # the outlet once more, so the stored state is the separate kernels'
             self.coarse.apply_bc(self._plan_c.pre.bc, self.even_c, stream=stream)
@@ -472,13 +492,14 @@ class RefinedStepper:
         if self._plan_c is not None:
             p = self._plan_c
             edge = int(self.coarse.dims[0] % 64 != 0)  # outlet nodes whose neighbour is in another wavefront
-            return 2 * (1 + len(self.fine_bcs)) + 1 + edge + len(p.residual_post) + len(p.residual_pre) + 2
+            return 2 * (1 + len(self.fine_bcs)) + 1 + edge + len(p.residual_post) + len(p.residual_pre) + \
+                (1 if self._one_interface else 2)
         if self.merged:
             sets = (self._set_post_both, self._set_pre_both, self._set_post_fine, self._set_pre_fine)
             rest = 2 * (len(self._f_post_rest) + len(self._f_pre_rest)) + len(self._c_post_rest) + len(self._c_pre_rest)
             return 2 + sum(s.handle is not None for s in sets) + rest + (1 if self._one_interface else 2)
         turb = int(self.collision == "k17" and self.coarse.turbulence == "amd")
-        return 2 * (1 + turb + len(self.fine_bcs)) + (1 + turb + len(self.coarse_bcs)) + 2
+        return 2 * (1 + turb + len(self.fine_bcs)) + (1 + turb + len(self.coarse_bcs)) + (1 if self._one_interface else 2)
 
     @property
     def lups_per_step(self) -> int:
