@@ -803,10 +803,10 @@ static vfx_status energy(const vfx_lattice* lat, bool enstrophy, const double* d
     if (!drho || !vx || !vy || !vz || !workspace || !out2) return fail(VFX_EINVAL, "NULL field/workspace/output");
     hipStream_t st = (hipStream_t)stream;
     const uint32_t nb = vfx::reduce_blocks(L.N);
-    if (enstrophy)
-        hipLaunchKernelGGL((vfx::k_reduce_energy<true>), dim3(nb), dim3(vfx::kRedBlock), 0, st, L, drho, vx, vy, vz, workspace);
-    else
-        hipLaunchKernelGGL((vfx::k_reduce_energy<false>), dim3(nb), dim3(vfx::kRedBlock), 0, st, L, drho, vx, vy, vz, workspace);
+    const bool plain = !L.solid && L.N * sizeof(double) < (1ull << 32);
+    auto* kernel = enstrophy ? (plain ? vfx::k_reduce_energy<true, true> : vfx::k_reduce_energy<true, false>)
+                             : (plain ? vfx::k_reduce_energy<false, true> : vfx::k_reduce_energy<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(vfx::kRedBlock), 0, st, L, drho, vx, vy, vz, workspace);
     hipLaunchKernelGGL((vfx::k_reduce_finish<2>), dim3(1), dim3(vfx::kRedBlock), 0, st, workspace, nb, out2);
     return hip_status(hipGetLastError(), enstrophy ? "enstrophy launch" : "kinetic energy launch");
 }

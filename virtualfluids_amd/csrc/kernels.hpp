@@ -947,14 +947,48 @@ template <int NV> __global__ void __launch_bounds__(kRedBlock) k_reduce_finish(c
         for (int c = 0; c < NV; ++c) out[c] = acc[c];
 }
 
-// Structured-box neighbour along one axis (periodic index wrap), -1 if solid.
-__device__ __forceinline__ int64_t fluid_nbr(const Lat& L, uint32_t x, uint32_t y, uint32_t z, int ax, int step)
+// The nodes up to R steps from node k along one axis of extent n and the given
+// stride (periodic index wrap, also for boxes smaller than the stencil), c the
+// node's coordinate.
+template <int R> struct AxisNodes {
+    uint32_t p[R + 1], m[R + 1];
+    __device__ __forceinline__ AxisNodes(uint32_t k, uint32_t c, uint32_t n, uint32_t stride)
+    {
+        const uint32_t back = (n - 1u) * stride;
+        uint32_t cp = c, cm = c;
+        p[0] = m[0] = k;
+#pragma unroll
+        for (int s = 1; s <= R; ++s) {
+            const bool wp = cp + 1u == n, wm = cm == 0u;
+            p[s] = wp ? p[s - 1] - back : p[s - 1] + stride;
+            m[s] = wm ? m[s - 1] + back : m[s - 1] - stride;
+            cp = wp ? 0u : cp + 1u;
+            cm = wm ? n - 1u : cm - 1u;
+        }
+    }
+};
+// order of the central difference at the node: 8, or 6 / 4 / 2 where the stencil
+// meets a solid node
+__device__ __forceinline__ int stencil_order(const Lat& L, const AxisNodes<4>& a)
 {
-    int64_t c[3] = {x, y, z};
-    const int64_t n[3] = {L.nx, L.ny, L.nz};
-    c[ax] = ((c[ax] + step) % n[ax] + n[ax]) % n[ax];
-    const uint32_t k = (uint32_t)(c[0] + n[0] * (c[1] + n[1] * c[2]));
-    return is_solid(L, k) ? -1 : (int64_t)k;
+    if (!L.solid) return 8;
+    if (is_solid(L, a.p[2]) || is_solid(L, a.m[2])) return 2;
+    if (is_solid(L, a.p[3]) || is_solid(L, a.m[3])) return 4;
+    return is_solid(L, a.p[4]) || is_solid(L, a.m[4]) ? 6 : 8;
+}
+// 280 times the derivative of order 8; W32: the fields' byte offsets fit 32 bits
+template <bool W32> __device__ __forceinline__ double derivative8(const double* v, const AxisNodes<4>& a)
+{
+    auto d = [&](int s) { return W32 ? elem(v, a.p[s]) - elem(v, a.m[s]) : v[a.p[s]] - v[a.m[s]]; };
+    return (28.0 * 8.0) * d(1) - (7.0 * 8.0) * d(2) + (8.0 * 4.0 * (1.0 / 3.0)) * d(3) - d(4);
+}
+__device__ __forceinline__ double derivative(const double* v, const AxisNodes<4>& a, int order)
+{
+    auto d = [&](int s) { return v[a.p[s]] - v[a.m[s]]; };
+    if (order == 8) return derivative8<false>(v, a) / (7.0 * 10.0 * 4.0);
+    if (order == 2) return d(1) / 2.0;
+    if (order == 4) return ((8.0 * v[a.p[1]] - 8.0 * v[a.m[1]]) - d(2)) / 12.0;
+    return ((5.0 * 9.0) * d(1) - 9.0 * d(2) + d(3)) / (6.0 * 10.0);
 }
 
 // Kinetic energy 1/2 rho |u|^2 summed over fluid nodes whose six axis
@@ -962,54 +996,61 @@ __device__ __forceinline__ int64_t fluid_nbr(const Lat& L, uint32_t x, uint32_t 
 // Enstrophy 1/2 rho |curl u|^2 on the same nodes with central differences of
 // order 8, reduced to 6/4/2 where the stencil meets a wall
 // (EnstrophyAnalyzer.cu:134-336).
-template <bool ENSTROPHY>
+//
+// The neighbours of an axis are stepped to (compare, select, add) and shared by
+// the two fields differentiated along it, and the chunks of an XCD are
+// contiguous, so the enstrophy stencil's rows and planes are found in its L2.
+// MI355X, 160^3: enstrophy 218 -> 97 us (one 64-bit remainder per neighbour and
+// field and chunks round robin before), 48 loads of 8 bytes per node and ~41 us
+// of L1 throughput; with the 64-bit offsets and order branches of the general
+// form 136.  Kinetic energy 29 -> 28 us, a stream of the four fields (26 at 5 TB/s).
+// PLAIN: no solid nodes and fields below 4 GiB (byte offsets of 32 bits).
+template <bool ENSTROPHY, bool PLAIN>
 __global__ void __launch_bounds__(kRedBlock) k_reduce_energy(Lat L, const double* rho, const double* vx, const double* vy,
                                                              const double* vz, double* partial)
 {
     double acc[2] = {0, 0};
+    const uint32_t full = gridDim.x / kXcds * kXcds;
+    const uint32_t chunk = ENSTROPHY && blockIdx.x < full ? xcd_slab(blockIdx.x, full) : blockIdx.x;
     for (int j = 0; j < kRedPerThread; ++j) {
-        const uint64_t i = (uint64_t)blockIdx.x * kRedChunk + (uint64_t)j * kRedBlock + threadIdx.x;
+        const uint64_t i = (uint64_t)chunk * kRedChunk + (uint64_t)j * kRedBlock + threadIdx.x;
         if (i >= L.N) continue;
         const uint32_t k = (uint32_t)i;
-        if (is_solid(L, k)) continue;
-        const uint32_t x = k % L.nx, r = k / L.nx, y = r % L.ny, z = r / L.ny;
-        bool ok = true;
-        for (int ax = 0; ax < 3 && ok; ++ax)
-            if (fluid_nbr(L, x, y, z, ax, 1) < 0 || fluid_nbr(L, x, y, z, ax, -1) < 0) ok = false;
-        if (!ok) continue;
-        if (!ENSTROPHY) {
-            acc[0] += 0.5 * (vx[k] * vx[k] + vy[k] * vy[k] + vz[k] * vz[k]) * (rho[k] + 1.0);
-            acc[1] += 1.0;
+        if (!PLAIN && is_solid(L, k)) continue;
+        const uint32_t r = fastdiv(k, L.div_x), x = k - r * L.nx, z = fastdiv(r, L.div_y), y = r - z * L.ny;
+        constexpr int R = ENSTROPHY ? 4 : 1;
+        const AxisNodes<R> ax(k, x, L.nx, 1u), ay(k, y, L.ny, L.nx), az(k, z, L.nz, L.nx * L.ny);
+        if (!PLAIN && L.solid &&
+            (is_solid(L, ax.p[1]) || is_solid(L, ax.m[1]) || is_solid(L, ay.p[1]) || is_solid(L, ay.m[1]) ||
+             is_solid(L, az.p[1]) || is_solid(L, az.m[1])))
             continue;
-        }
-        // derivative of field v along axis ax at node k
-        auto deriv = [&](const double* v, int ax) {
-            int order = 8;
-            int64_t p[5], m[5];
-            for (int s = 1; s <= 4; ++s) {
-                p[s] = fluid_nbr(L, x, y, z, ax, s);
-                m[s] = fluid_nbr(L, x, y, z, ax, -s);
-            }
-            if (p[2] < 0 || m[2] < 0) order = 2;
-            if ((p[3] < 0 || m[3] < 0) && order > 4) order = 4;
-            if ((p[4] < 0 || m[4] < 0) && order > 6) order = 6;
-            auto d = [&](int s) { return v[p[s]] - v[m[s]]; };
-            if (order == 2) return d(1) / 2.0;
-            if (order == 4) return ((8.0 * v[p[1]] - 8.0 * v[m[1]]) - d(2)) / 12.0;
-            if (order == 6) return ((5.0 * 9.0) * d(1) - 9.0 * d(2) + d(3)) / (6.0 * 10.0);
-            return ((28.0 * 8.0) * d(1) - (7.0 * 8.0) * d(2) + (8.0 * 4.0 * (1.0 / 3.0)) * d(3) - d(4)) / (7.0 * 10.0 * 4.0);
-        };
-        const double dyvz = deriv(vz, 1), dzvy = deriv(vy, 2);
-        const double dzvx = deriv(vx, 2), dxvz = deriv(vz, 0);
-        const double dxvy = deriv(vy, 0), dyvx = deriv(vx, 1);
-        const double wx = dyvz - dzvy, wy = dzvx - dxvz, wz = dxvy - dyvx;
-        acc[0] += 0.5 * (rho[k] + 1.0) * (wx * wx + wy * wy + wz * wz);
         acc[1] += 1.0;
+        if constexpr (!ENSTROPHY) {
+            acc[0] += 0.5 * (vx[k] * vx[k] + vy[k] * vy[k] + vz[k] * vz[k]) * (rho[k] + 1.0);
+            continue;
+        } else {
+            if constexpr (!PLAIN) {
+                const int ox = stencil_order(L, ax), oy = stencil_order(L, ay), oz = stencil_order(L, az);
+                if (ox != 8 || oy != 8 || oz != 8) {
+                    const double dyvz = derivative(vz, ay, oy), dzvy = derivative(vy, az, oz);
+                    const double dzvx = derivative(vx, az, oz), dxvz = derivative(vz, ax, ox);
+                    const double dxvy = derivative(vy, ax, ox), dyvx = derivative(vx, ay, oy);
+                    const double wx = dyvz - dzvy, wy = dzvx - dxvz, wz = dxvy - dyvx;
+                    acc[0] += 0.5 * (rho[k] + 1.0) * (wx * wx + wy * wy + wz * wz);
+                    continue;
+                }
+            }
+            // one division for the six derivatives
+            const double wx = derivative8<PLAIN>(vz, ay) - derivative8<PLAIN>(vy, az);
+            const double wy = derivative8<PLAIN>(vx, az) - derivative8<PLAIN>(vz, ax);
+            const double wz = derivative8<PLAIN>(vy, ax) - derivative8<PLAIN>(vx, ay);
+            acc[0] += 0.5 * (rho[k] + 1.0) * (wx * wx + wy * wy + wz * wz) / (280.0 * 280.0);
+        }
     }
     block_sum<2>(acc);
     if (threadIdx.x == 0) {
-        partial[(uint64_t)blockIdx.x * 2] = acc[0];
-        partial[(uint64_t)blockIdx.x * 2 + 1] = acc[1];
+        partial[(uint64_t)chunk * 2] = acc[0];
+        partial[(uint64_t)chunk * 2 + 1] = acc[1];
     }
 }
 
@@ -2121,33 +2162,62 @@ namespace vfx {
 // direction d = slot^-1(p) (p itself at even parity, inv(p) at odd), which
 // fixes the FP16 scale and reference offset; FP32/FP64 storage is copied.
 // Export writes NaN as 0, as serialize does.
+// blockIdx.y is the plane: its direction, scale and offset are wave-uniform and
+// no element divides its index by the node count (a 64-bit division, ~100
+// instructions per element before).  MI355X, 160^3 FP32 to float, 885 MB: 201 ->
+// 162 us with four elements per thread, 236 with one (432 000 workgroups).
+template <typename S> struct PlaneScale {
+    int d;
+    float ld, st, sh, ss;
+    __device__ __forceinline__ PlaneScale(const Lat& L, int p, bool even)
+    {
+        d = 0;
+        ld = st = 1.f;
+        sh = ss = 0.f;
+        if constexpr (sizeof(S) == 2) {
+            // constant-index selects: the kernel argument arrays stay in place
+#pragma unroll
+            for (int e = 0; e < 27; ++e)
+                if (p == slot(e, even)) {
+                    d = e;
+                    ld = L.ld[weight_class(e)];
+                    st = L.st[weight_class(e)];
+                    sh = L.sh[e];
+                    ss = L.ss[e];
+                }
+        }
+    }
+};
+constexpr uint32_t kCopyPerThread = 4; // elements per thread, loaded before the first is stored
 template <typename S, bool EVEN, typename O>
 __global__ void __launch_bounds__(256) k_export(Lat L, O* out)
 {
     using T = typename Compute<S>::T;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    const uint64_t n = 27ull * L.N;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const int p = (int)(i / L.N);
-        const uint32_t j = (uint32_t)(i - (uint64_t)p * L.N);
-        const int d = EVEN ? p : inv(p);
-        T v = Storage<S, T>::ld(plane<S>(L, p), j, L.ld[weight_class(d)], L.sh[d]);
-        if (v != v) v = T(0);
-        out[i] = (O)v;
-    }
+    const int p = (int)blockIdx.y;
+    const PlaneScale<S> c(L, p, EVEN);
+    const uint32_t n = (uint32_t)L.N, j0 = blockIdx.x * (256u * kCopyPerThread) + threadIdx.x;
+    T v[kCopyPerThread];
+#pragma unroll
+    for (uint32_t u = 0; u < kCopyPerThread; ++u)
+        if (j0 + u * 256u < n) v[u] = Storage<S, T>::ld(plane<S>(L, p), j0 + u * 256u, c.ld, c.sh);
+#pragma unroll
+    for (uint32_t u = 0; u < kCopyPerThread; ++u)
+        if (j0 + u * 256u < n) (out + (uint64_t)p * L.N)[j0 + u * 256u] = v[u] != v[u] ? O(0) : (O)v[u];
 }
 template <typename S, bool EVEN, typename O>
 __global__ void __launch_bounds__(256) k_import(Lat L, const O* in)
 {
     using T = typename Compute<S>::T;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    const uint64_t n = 27ull * L.N;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const int p = (int)(i / L.N);
-        const uint32_t j = (uint32_t)(i - (uint64_t)p * L.N);
-        const int d = EVEN ? p : inv(p);
-        Storage<S, T>::st(plane<S>(L, p), j, (T)in[i], L.st[weight_class(d)], L.ss[d]);
-    }
+    const int p = (int)blockIdx.y;
+    const PlaneScale<S> c(L, p, EVEN);
+    const uint32_t n = (uint32_t)L.N, j0 = blockIdx.x * (256u * kCopyPerThread) + threadIdx.x;
+    O v[kCopyPerThread];
+#pragma unroll
+    for (uint32_t u = 0; u < kCopyPerThread; ++u)
+        if (j0 + u * 256u < n) v[u] = (in + (uint64_t)p * L.N)[j0 + u * 256u];
+#pragma unroll
+    for (uint32_t u = 0; u < kCopyPerThread; ++u)
+        if (j0 + u * 256u < n) Storage<S, T>::st(plane<S>(L, p), j0 + u * 256u, (T)v[u], c.st, c.ss);
 }
 
 // ------------------------------------------------------- AMD viscosity ----
@@ -2167,9 +2237,9 @@ __device__ __forceinline__ void amd_derivatives(uint32_t k, uint32_t km, uint32_
     const T div = (fm && fp) ? T(0.5) : T(1);
     kp = fp ? kp : k;
     km = fm ? km : k;
-    dvx = (elem(vx, kp) - elem(vx, km)) * div;
-    dvy = (elem(vy, kp) - elem(vy, km)) * div;
-    dvz = (elem(vz, kp) - elem(vz, km)) * div;
+    dvx = (vx[kp] - vx[km]) * div;
+    dvy = (vy[kp] - vy[km]) * div;
+    dvz = (vz[kp] - vz[km]) * div;
 }
 
 // Bound by its reads past L2: with the blocks round robin over the XCDs the rows
@@ -2177,7 +2247,8 @@ __device__ __forceinline__ void amd_derivatives(uint32_t k, uint32_t km, uint32_
 // again, five times the fields' bytes.  With a contiguous eighth of the lattice
 // per XCD (xcd_slab) they are in its own: 224x144x120 33.6 -> 22.0 us (MI355X;
 // 62 MB that it must move, 12 us).  Selecting a neighbour by its index, once for
-// the three components, and 32-bit element offsets alone changed nothing.
+// the three components, alone changed nothing.  (The fields are float beside
+// 2-byte populations too: a 32-bit byte offset would not reach every node.)
 template <typename T> __global__ void __launch_bounds__(256) k_turb_amd(Lat L, int direct, T C)
 {
     const uint32_t k = xcd_slab(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
@@ -2466,8 +2537,7 @@ template <typename S> hipError_t launch_rw(const Lat& L, int direct, bool even, 
 template <typename S>
 hipError_t launch_vf_array(const Lat& L, bool even, bool fp64, void* out, const void* in, hipStream_t st)
 {
-    const uint64_t n = 27ull * L.N;
-    const unsigned g = (unsigned)std::min<uint64_t>((n + kBlock - 1) / kBlock, 65536), b = kBlock;
+    const dim3 g(grid_for(L.N, kBlock * kCopyPerThread), 27), b(kBlock);
     if (out) {
         if (fp64) {
             if (even) hipLaunchKernelGGL((k_export<S, true, double>), g, b, 0, st, L, (double*)out);
