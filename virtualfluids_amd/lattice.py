@@ -258,13 +258,17 @@ class Lattice:
         self.forces = tuple(float(x) for x in forces)
         self.force_factor = float(force_factor)
 
-    def collide_stream(self, collision="k17", even=True, write_macro=False, stream=None, apply_body_force=False):
+    def _template(self, write_macro, apply_body_force):
+        """The collision template; makes the fields it writes."""
         if write_macro:
             self._alloc_macro()
         if apply_body_force and self.body_force is None:
             raise ValueError("apply_body_force needs set_body_force first")
-        tmpl = (V.VFX_TEMPLATE_ALL_FEATURES if write_macro else V.VFX_TEMPLATE_APPLY_BODY_FORCE) if apply_body_force \
+        return (V.VFX_TEMPLATE_ALL_FEATURES if write_macro else V.VFX_TEMPLATE_APPLY_BODY_FORCE) if apply_body_force \
             else (V.VFX_TEMPLATE_WRITE_MACRO if write_macro else V.VFX_TEMPLATE_DEFAULT)
+
+    def collide_stream(self, collision="k17", even=True, write_macro=False, stream=None, apply_body_force=False):
+        tmpl = self._template(write_macro, apply_body_force)
         s = self.struct()
         V.check(V.lib().vfx_collide_stream(C.byref(s), COLLISION[collision], int(bool(even)), tmpl, _stream(stream)),
                 "vfx_collide_stream")
@@ -286,7 +290,7 @@ class Lattice:
         s = self.struct()
         V.check(V.lib().vfx_turbulent_viscosity_amd(C.byref(s), _stream(stream)), "vfx_turbulent_viscosity_amd")
 
-    def apply_bc(self, bc: "BoundaryCondition", even=True, stream=None):
+    def _check_bc(self, bc: "BoundaryCondition"):
         if bc.max_node >= self.n_nodes:
             raise ValueError("boundary node index out of range")
         if bc.wm is not None:
@@ -295,6 +299,9 @@ class Lattice:
             self._alloc_macro()
         if bc.precursor is not None and bc.precursor.real != self._macro_dtype():
             raise ValueError("precursor weights and planes must have the lattice's arithmetic type")
+
+    def apply_bc(self, bc: "BoundaryCondition", even=True, stream=None):
+        self._check_bc(bc)
         s = self.struct()
         b = bc.struct(self._macro_dtype())
         V.check(V.lib().vfx_bc_apply(C.byref(s), C.byref(b), int(bool(even)), _stream(stream)), "vfx_bc_apply")
@@ -976,50 +983,76 @@ class Stepper:
                     self.lattice.apply_bc(bc, self.even, stream=stream)
         self._primed = True
 
+    def _bc_call(self, bc, s, stream):
+        """bc's launch as a function of the parity, for the steps of one call:
+        the tables are handed over once (lattice view s).  Precursor planes
+        rotate, so those make a new view every step."""
+        lat = self.lattice
+        lat._check_bc(bc)
+        if bc.precursor is not None:
+            def precursor(even):
+                if bc.precursor.reader is not None:
+                    bc.precursor.advance(self.t, stream)
+                lat.apply_bc(bc, even, stream=stream)
+            return precursor
+        b = bc.struct(lat._macro_dtype())
+        apply, st = V.lib().vfx_bc_apply, _stream(stream)
+        args = C.byref(s), C.byref(b)
+        return lambda even: V.check(apply(*args, int(even), st), "vfx_bc_apply")
+
     def _step_fused(self, n, stream):
         plan = self.fused_plan()
         lat = self.lattice
         self._prime(stream)
+        if n <= 0:
+            return
+        s = lat.struct()
+        post = [self._bc_call(bc, s, stream) for bc in plan.residual_post]
+        pre = [self._bc_call(bc, s, stream) for bc in plan.residual_pre]
         for i in range(n):
             # the pressure group of the previous step of this run is applied
             # while the node's populations are gathered
             lat.k17_step_fused(self.even, plan.post, plan.pre, apply_pre=i > 0, any_mask=plan.any_mask,
                                stream=stream)
-            for bc in plan.residual_post:
-                if bc.precursor is not None and bc.precursor.reader is not None:
-                    bc.precursor.advance(self.t, stream)
-                lat.apply_bc(bc, self.even, stream=stream)
+            for run in post:
+                run(self.even)
             self.t += 1
             self.even = not self.even
-            for bc in plan.residual_pre:
-                lat.apply_bc(bc, self.even, stream=stream)
+            for run in pre:
+                run(self.even)
         # leave the populations as the separate kernels would
-        if n > 0 and plan.pre is not None:
+        if plan.pre is not None:
             lat.apply_bc(plan.pre.bc, self.even, stream=stream)
 
     def step(self, n=1, stream=None):
         if self.fuse:
             return self._step_fused(n, stream)
         self._prime(stream)
-        # precursor inflows run last among the post-collision conditions (UpdateGrid27.cpp:252)
-        post = [b for b in self.bcs if not b.pre_collision and b.kind not in BoundaryCondition.PRECURSOR] + \
-               [b for b in self.bcs if b.kind in BoundaryCondition.PRECURSOR]
-        pre = [b for b in self.bcs if b.pre_collision]
+        if n <= 0:
+            return
+        lat = self.lattice
         # wall models sample the velocities the collision writes
         write_macro = any(getattr(b, "wm", None) is not None for b in self.bcs)
+        tmpl = lat._template(write_macro, self.apply_body_force)
+        # the lattice and its tables are handed over once per call, not once per
+        # launch: a small lattice's step takes less time than making the views
+        s = lat.struct()
+        # precursor inflows run last among the post-collision conditions (UpdateGrid27.cpp:252)
+        order = sorted(self.bcs, key=lambda b: b.kind in BoundaryCondition.PRECURSOR)
+        post = [self._bc_call(b, s, stream) for b in order if not b.pre_collision]
+        pre = [self._bc_call(b, s, stream) for b in self.bcs if b.pre_collision]
+        L, st, view, coll = V.lib(), _stream(stream), C.byref(s), COLLISION[self.collision]
+        amd = self.collision == "k17" and getattr(lat, "turbulence", "none") == "amd"
         for _ in range(n):
-            self.lattice.collide_stream(self.collision, self.even, write_macro=write_macro, stream=stream,
-                                        apply_body_force=self.apply_body_force)
-            for bc in post:
-                if bc.precursor is not None and bc.precursor.reader is not None:
-                    bc.precursor.advance(self.t, stream)
-                self.lattice.apply_bc(bc, self.even, stream=stream)
+            V.check(L.vfx_collide_stream(view, coll, int(self.even), tmpl, st), "vfx_collide_stream")
+            for run in post:
+                run(self.even)
             self.t += 1
             self.even = not self.even
-            if self.collision == "k17" and getattr(self.lattice, "turbulence", "none") == "amd":
-                self.lattice.turbulent_viscosity_amd(stream=stream)
-            for bc in pre:
-                self.lattice.apply_bc(bc, self.even, stream=stream)
+            if amd:
+                V.check(L.vfx_turbulent_viscosity_amd(view, st), "vfx_turbulent_viscosity_amd")
+            for run in pre:
+                run(self.even)
 
     def populations(self) -> torch.Tensor:
         return self.lattice.read_populations(self.even)
