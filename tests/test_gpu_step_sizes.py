@@ -1,5 +1,5 @@
 """The structured step on boxes whose rows, slabs and node count do not fit its
-tiles or wavefronts, against the CPU checker: FP64 reproduces it bit for bit.
+tiles or wavefronts, against the oracle: FP64 reproduces it bit for bit.
 The sizes sit at the edges of the flat node mapping (one node in a direction,
 rows of one node more or less than a wavefront, a last tile of one node)."""
 import numpy as np
