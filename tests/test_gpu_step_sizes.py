@@ -36,7 +36,7 @@ def test_fp16_models_reduced_form_equals_the_reference_order(cuda, model, sparse
     of ~1500 operations (1e-5 of the largest population, generous) plus one unit
     of the half it is stored in (2^-10 of the population itself).  The eddy
     viscosity is compared with FP64's from the same populations: the reduced
-    form is at most half as far off again as the reference order."""
+    form is no further off than the reference order."""
     print(f"[fp16 {model} {sparse}]", flush=True)
     dims = (37, 11, 8)
     n = int(np.prod(dims))
@@ -65,5 +65,27 @@ def test_fp16_models_reduced_form_equals_the_reference_order(cuda, model, sparse
         out.append((lat.f.double().cpu().numpy().reshape(27, n), lat.nut.double().cpu().numpy()))
     (a, va), (b, vb), (_, v) = out
     assert np.all(np.abs(a - b) <= 1e-5 * np.abs(b).max(axis=1, keepdims=True) + 2.0 ** -10 * np.abs(b))
-    assert np.linalg.norm(va - v) <= 1.5 * np.linalg.norm(vb - v)
+    assert np.linalg.norm(va - v) <= np.linalg.norm(vb - v)
     assert not np.array_equal(a, b)  # the two forms did run
+
+
+@pytest.mark.parametrize("model", ["smagorinsky", "qr", "amd"])
+@pytest.mark.parametrize("dims", [(37, 11, 8), (65, 16, 9)])
+def test_fp16_models_write_the_reference_orders_density_and_velocity(cuda, model, dims):
+    """The 32-bit fields the collision writes, and the viscosity the AMD kernel
+    forms from them, are the same bits in the default and the "plain" variant."""
+    print(f"[fp16 fields {model} {dims}]", flush=True)
+    n = int(np.prod(dims))
+    out = []
+    for variant in ("default", "plain"):
+        lat = vfx.Lattice(dims, storage="fp16", omega=1.95, turbulence=model, sgs_constant=0.2, variant=variant)
+        lat.init_equilibrium(*cases.random_flow(dims, seed=9))
+        lat.nut.copy_(torch.from_numpy(1e-3 * (1.0 + np.sin(np.arange(n)))).to(lat.nut.dtype))
+        lat.collide_stream("k17", True, write_macro=True)
+        fields = list(lat.macro)
+        if model == "amd":
+            lat.turbulent_viscosity_amd()
+            fields.append(lat.nut)
+        out.append(fields)
+    for a, b in zip(*out):
+        assert torch.equal(a, b)

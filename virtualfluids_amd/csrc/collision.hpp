@@ -577,7 +577,8 @@ __device__ __forceinline__ void node_rates(const Rates<float>& R0, float nut, Ra
 // OUTER2: run the backward sweeps with bwdf2, so that population d leaves
 // scaled by 2^weight_class(d) (the caller's store removes the factor; used
 // where the store multiplies by a scale anyway, i.e. FP16 storage).
-// TM: eddy-viscosity model; the node's rates then come from its own omega.
+// TM: eddy-viscosity model; the node's rates then come from its own omega, and
+// density and velocity are k17's bits.
 template <bool OUTER2, int TM = kTurbNone>
 __device__ __forceinline__ void k17_fast(float (&m)[27], const Rates<float>& R0, float (&mv)[4], float& nut)
 {
@@ -591,6 +592,8 @@ __device__ __forceinline__ void k17_fast(float (&m)[27], const Rates<float>& R0,
     // depend on the velocity), so its sums ys, yd, ym per x plane are formed
     // here too: drho = (ym0 + ym2) + ym1 and jx = ym2 - ym0 are the sums of the
     // x sweep's first line, jy = sum of yd; jz sums the nine z differences.
+    float rs, js[3];
+    if constexpr (TM != kTurbNone) pyramid_sums(m, rs, js[0], js[1], js[2]);
     float zs[3][3], zd[3][3], zm[3][3];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -609,13 +612,24 @@ __device__ __forceinline__ void k17_fast(float (&m)[27], const Rates<float>& R0,
     }
     const float xs = ym[0] + ym[2];
     const float jx = ym[2] - ym[0];
-    const float drho = xs + ym[1];
-    const float jy = (yd[0] + yd[2]) + yd[1];
-    const float jz = (((zd[0][0] + zd[2][2]) + (zd[0][2] + zd[2][0])) + ((zd[0][1] + zd[2][1]) + (zd[1][0] + zd[1][2]))) + zd[1][1];
-    const float oneOverRho = rcpf(drho + 1.f);
-    const float vx = jx * oneOverRho + R.fx;
-    const float vy = jy * oneOverRho + R.fy;
-    const float vz = jz * oneOverRho + R.fz;
+    const float ms = xs + ym[1];
+    float drho, vx, vy, vz, oneOverRho;
+    if constexpr (TM != kTurbNone) {
+        // these are written as 32-bit fields, and the AMD viscosity is formed
+        // from them: summed and divided as in k17, so that they are its bits (the
+        // sweeps' density is 1.3 times as far off; +5% time, none beside AMD's
+        // kernel)
+        drho = rs, vx = js[0], vy = js[1], vz = js[2];
+        oneOverRho = 1.f / (drho + 1.f);
+    } else {
+        drho = ms, vx = jx;
+        vy = (yd[0] + yd[2]) + yd[1];
+        vz = (((zd[0][0] + zd[2][2]) + (zd[0][2] + zd[2][0])) + ((zd[0][1] + zd[2][1]) + (zd[1][0] + zd[1][2]))) + zd[1][1];
+        oneOverRho = rcpf(drho + 1.f);
+    }
+    vx = vx * oneOverRho + R.fx;
+    vy = vy * oneOverRho + R.fy;
+    vz = vz * oneOverRho + R.fz;
     const float vx2 = vx * vx, vy2 = vy * vy, vz2 = vz * vz;
     const float tx = 2.f * vx, ty = 2.f * vy, tz = 2.f * vz;
 
@@ -636,7 +650,7 @@ __device__ __forceinline__ void k17_fast(float (&m)[27], const Rates<float>& R0,
         fwdf<2>(VFX_M(i, 0, 1), VFX_M(i, 1, 1), VFX_M(i, 2, 1), vy, vy2, ty, 0.f);
         fwdf<1>(VFX_M(i, 0, 2), VFX_M(i, 1, 2), VFX_M(i, 2, 2), vy, vy2, ty, wv[i] * c1o3);
     }
-    fwdf_sums<2>(VFX_M(0, 0, 0), VFX_M(1, 0, 0), VFX_M(2, 0, 0), xs, jx, drho, vx, vx2, tx, 1.f);
+    fwdf_sums<2>(VFX_M(0, 0, 0), VFX_M(1, 0, 0), VFX_M(2, 0, 0), xs, jx, ms, vx, vx2, tx, 1.f);
     fwdf<2>(VFX_M(0, 1, 0), VFX_M(1, 1, 0), VFX_M(2, 1, 0), vx, vx2, tx, 0.f);
     fwdf<2>(VFX_M(0, 0, 1), VFX_M(1, 0, 1), VFX_M(2, 0, 1), vx, vx2, tx, 0.f);
     fwdf<1>(VFX_M(0, 2, 0), VFX_M(1, 2, 0), VFX_M(2, 2, 0), vx, vx2, tx, c1o3);

@@ -2351,13 +2351,16 @@ hipError_t launch_step_t(const Lat& L, int direct, const Rates<typename Compute<
 // The reduced-operation form (FP32 arithmetic only) or the reference order.
 // With an eddy-viscosity model the reduced form runs on 2-byte storage only: the
 // reference order (rates of every node with IEEE divisions, ~1500 instructions)
-// is bound by its arithmetic there, the reduced one by memory (MI355X,
-// 224x144x120 with AMD: 175 -> 105 us per step, 810 -> 541 per 4 steps with the
-// viscosity kernel), and both sit at the storage's rounding (error of the
-// populations against 64 bits after 10 steps 3.0e-4 to 4.3e-4, equal to 0.3%,
-// omega 1.8 to 1.999, all models).  On 4-byte storage both are bound by memory
-// (256x160x100: 185 us) and the reduced form's error is up to twice the
-// reference order's (8.3e-7 against 4.4e-7), so that one keeps the latter.
+// is bound by its arithmetic there, the reduced one by memory (MI355X, us per
+// step, reference order -> reduced: Smagorinsky 224x144x120 169 -> 95,
+// 384x256x200 974 -> 489; AMD with its viscosity kernel 205 -> 129, 1086 ->
+// 627).  Density and velocity are the reference order's bits, the error of the
+// viscosity against 64 bits is 0.91 to 1.00 of its and that of the populations,
+// which is the storage's rounding, the same to four digits (one step from the
+// same populations, omega 1.8 to 1.999, all models).  On 4-byte storage both are
+// bound by memory (256x160x100: 185 us) and the populations of the reduced form
+// are up to twice as far off (8.3e-7 against 4.4e-7 after 10 steps), so that one
+// keeps the reference order.
 template <typename S, int COLL>
 hipError_t launch_step_p(const Lat& L, int direct, bool even, bool fast, const Rates<typename Compute<S>::T>& R,
                          hipStream_t st)
