@@ -37,3 +37,40 @@ def test_every_lane_gives_the_separate_kernels_bytes(cuda, nx, normal, storage):
         out.append(lat.f.view(torch.uint8))
     assert torch.equal(*out)
     assert n == lat.n_nodes
+
+
+def _call(lat, group, apply_pre):
+    st, real = lat.struct(), lat._macro_dtype()
+    g = group.struct(real)
+    C = vfx._lib.C
+    vfx.check(vfx.lib().vfx_k17_step_fused(C.byref(st), 1, None, 0, C.byref(g), None, apply_pre, None), "vfx_k17_step_fused")
+
+
+@pytest.mark.parametrize("storage", ["fp64", "fp32", "fp16"])
+@pytest.mark.parametrize("fault", ["neighbour", "mask", "base"])
+@pytest.mark.parametrize("normal", [1, 2])
+def test_malformed_entries_select_nothing_on_every_lane(cuda, normal, fault, storage):
+    """Entries whose neighbour is not the one beside them, or which the masks do
+    not hold, leave the plain step's bytes wherever they lie in a wavefront."""
+    print(f"[malformed {normal} {fault} {storage}]", flush=True)
+    dims = (70, 9, 8)
+    k = 70 * np.arange(72) + (68 if normal == 1 else 1)
+    assert np.any(k % 64 == (0 if normal == 1 else 63))
+    step = -1 if normal == 1 else 1
+    out = []
+    for malformed in (False, True):
+        lat = vfx.Lattice(dims, storage=storage, omega=1.9)
+        lat.init_equilibrium(*cases.random_flow(dims, seed=normal))
+        if malformed:
+            bc = vfx.BoundaryCondition(4, k, rho=1e-2 * np.ones(72), normal=normal,
+                                       neighbors=k + (2 * step if fault == "neighbour" else step))
+            g = vfx.FusedGroup(bc, lat.n_nodes)
+            if fault == "mask":
+                g.node_mask.zero_()
+            if fault == "base":
+                g.word_base += 1000
+            _call(lat, g, 1)
+        else:
+            lat.collide_stream("k17", True)
+        out.append(lat.f.view(torch.uint8))
+    assert torch.equal(*out)

@@ -1595,14 +1595,6 @@ __global__ void __launch_bounds__(256) k_bc_pressure(Lat L, BCDev B)
 {
     bc_pressure_entry<S, EVEN>(L, B, blockIdx.x * blockDim.x + threadIdx.x);
 }
-// the entries k_step_pre leaves out: nodes in the wavefront's first lane (last,
-// for an outward normal -x)
-template <typename S, bool EVEN>
-__global__ void __launch_bounds__(256) k_bc_pressure_edge(Lat L, BCDev B)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < B.n && (B.k[i] & 63u) == (B.normal == dP00 ? 0u : 63u)) bc_pressure_entry<S, EVEN>(L, B, i);
-}
 
 // Several boundary groups, possibly of different lattices of one storage
 // type, in one launch: block b runs the job whose block range holds b (jobs
@@ -1989,6 +1981,23 @@ __global__ void __launch_bounds__(256) k_step_pre(Lat L, Rates<typename Compute<
     if (!active) return;
     collide<T, VFX_K17, FAST, O2>(m, R, mv, nut);
     scatter_post<S, T, EVEN, O2>(L, kk, m);
+}
+
+// The entries k_step_pre leaves out: nodes in the wavefront's first lane (last,
+// for an outward normal -x), chosen by the same tables and conditions.
+template <typename S, bool EVEN>
+__global__ void __launch_bounds__(256) k_bc_pressure_edge(Lat L, FusedGroup gp)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= gp.B.n) return;
+    const bool px = gp.B.normal == dP00;
+    const uint32_t k = gp.B.k[i];
+    if ((k & 63u) != (px ? 0u : 63u) || k >= (uint32_t)L.N || is_solid(L, k)) return;
+    const uint32_t word = gp.mask[k >> 5], bit = 1u << (k & 31u);
+    if (!(word & bit) || gp.base[k >> 5] + (uint32_t)__builtin_popcount(word & (bit - 1u)) != i ||
+        gp.B.kn[i] != (px ? k - 1u : k + 1u))
+        return; // malformed tables select nothing
+    bc_pressure_entry<S, EVEN>(L, gp.B, i);
 }
 
 // The coarse step and the first fine step of a nest (or any two structured
@@ -2421,8 +2430,8 @@ hipError_t launch_step_fused(const Lat& L, bool even, double omega, const double
         const dim3 edge(grid_for(gp.B.n, kBlock)), b(kBlock);
         // rows of whole wavefronts keep the pair in one (the caller's x mod 64 condition)
         if (L.nx % 64u != 0) {
-            if (even) hipLaunchKernelGGL((k_bc_pressure_edge<S, true>), edge, b, 0, st, L, gp.B);
-            else hipLaunchKernelGGL((k_bc_pressure_edge<S, false>), edge, b, 0, st, L, gp.B);
+            if (even) hipLaunchKernelGGL((k_bc_pressure_edge<S, true>), edge, b, 0, st, L, gp);
+            else hipLaunchKernelGGL((k_bc_pressure_edge<S, false>), edge, b, 0, st, L, gp);
         }
         const unsigned tile = L.tile ? L.tile : sizeof(S) == 4 ? 128u : 256u;
         const dim3 g(grid_for(L.N, tile)), t(tile);
