@@ -320,10 +320,12 @@ typedef struct vfx_fused_bc {
  *    i.e. x mod 64 != 0 (!= 63): the replacement vfx_bc_apply makes after the
  *    previous step's parity flip is made inside this step, from the
  *    neighbour's populations the neighbouring lane gathers, which spares the
- *    cache lines a kernel of its own reads again (where nx is no multiple of
- *    64, a small launch before the step takes the nodes whose neighbour lies in
- *    another 64 consecutive node numbers) (apply_pre = 1;
- *    0 on the first step of a run, before which no pressure boundary ran).
+ *    cache lines a kernel of its own reads again.  apply_pre: 0 on the first
+ *    step of a run, before which no pressure boundary ran, else 1, or -1.  Where
+ *    nx is no multiple of 64, a node's neighbour may lie in another 64
+ *    consecutive node numbers (k mod 64 = 0, or 63 for dM00): with 1 a small
+ *    launch before the step looks for such nodes and takes them; -1 says that
+ *    the list has none, spares the launch and leaves them as they are.
  *    Until the next step the boundary nodes then hold the un-replaced
  *    populations: vfx_bc_apply(pre->bc) with the new parity gives the state
  *    the separate launches leave, before it is read;

@@ -74,3 +74,29 @@ def test_malformed_entries_select_nothing_on_every_lane(cuda, normal, fault, sto
             lat.collide_stream("k17", True)
         out.append(lat.f.view(torch.uint8))
     assert torch.equal(*out)
+
+
+@pytest.mark.parametrize("storage", ["fp64", "fp32", "fp16"])
+def test_without_the_launch_before_the_step(cuda, storage):
+    """apply_pre -1 takes every entry but the ones whose neighbour lies in another
+    wavefront; a group that has none is told so by itself."""
+    print(f"[no edge launch {storage}]", flush=True)
+    dims = (70, 9, 8)
+    k = 70 * np.arange(72) + 68
+    inside = k[k % 64 != 0]
+    assert 0 < inside.size < k.size
+    out = []
+    for fused in (False, True):
+        lat = vfx.Lattice(dims, storage=storage, omega=1.9)
+        lat.init_equilibrium(*cases.random_flow(dims, seed=3))
+        nodes = k if fused else inside
+        bc = vfx.BoundaryCondition(4, nodes, rho=1e-2 * np.cos(nodes), neighbors=nodes - 1, normal=1)
+        if fused:
+            g = vfx.FusedGroup(bc, lat.n_nodes)
+            assert g.edge and not vfx.FusedGroup(bc.subset(np.flatnonzero(k % 64)), lat.n_nodes).edge
+            _call(lat, g, -1)
+        else:
+            lat.apply_bc(bc, True)
+            lat.collide_stream("k17", True)
+        out.append(lat.f.view(torch.uint8))
+    assert torch.equal(*out)

@@ -552,7 +552,7 @@ vfx_status vfx_k17_step_fused(const vfx_lattice* lat, int32_t is_even, const vfx
     if (vfx_status s = fused_inputs(lat, post, n_post, pre, L, g)) return s;
     hipStream_t st = (hipStream_t)stream;
     hipError_t e;
-    const int ap = apply_pre != 0;
+    const int ap = apply_pre == -1 ? -1 : apply_pre != 0;
     const double* lim = lat->quadric_limiter;
     switch (lat->storage) {
     case VFX_FP64:

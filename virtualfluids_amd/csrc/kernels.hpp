@@ -1941,8 +1941,10 @@ __device__ __forceinline__ void fused_pressure(const Lat& L, const FusedGroup& G
 // the step schedules worse, 190 us); the group's words are read before the
 // populations, the entry while they arrive (after them: 150 us).  A boundary
 // node whose neighbour is in another wavefront (lane 0, or 63 for -x) is left to
-// k_bc_pressure_edge, launched before.  MI355X, FP16 channel 288x144x144: 135 us
-// + 4.6 for the edge, against 123 + 32 for the plain step and k_bc_pressure.
+// k_bc_pressure_edge, launched before where the list has one.  MI355X, us per
+// step, FP16: channel 288x144x144 143 against 129 + 33 for the plain step and
+// k_bc_pressure (160 in turn), 230x130x120 with 472 of 15104 entries in the edge
+// launch 81 + 6.3 against 70 + 16.
 template <typename S, bool EVEN>
 __global__ void __launch_bounds__(256) k_step_pre(Lat L, Rates<typename Compute<S>::T> R, FusedGroup gp)
 {
@@ -1984,7 +1986,9 @@ __global__ void __launch_bounds__(256) k_step_pre(Lat L, Rates<typename Compute<
 }
 
 // The entries k_step_pre leaves out: nodes in the wavefront's first lane (last,
-// for an outward normal -x), chosen by the same tables and conditions.
+// for an outward normal -x), chosen by the same tables and conditions.  Not
+// launched for lists without such nodes (every x in a row has one k mod
+// gcd(nx, 64)): 144.5 -> 143.2 us per step of the 288x144x144 channel.
 template <typename S, bool EVEN>
 __global__ void __launch_bounds__(256) k_bc_pressure_edge(Lat L, FusedGroup gp)
 {
@@ -2428,8 +2432,9 @@ hipError_t launch_step_fused(const Lat& L, bool even, double omega, const double
     hipError_t e = hipSuccess;
     if (gp.mask && apply_pre) {
         const dim3 edge(grid_for(gp.B.n, kBlock)), b(kBlock);
-        // rows of whole wavefronts keep the pair in one (the caller's x mod 64 condition)
-        if (L.nx % 64u != 0) {
+        // rows of whole wavefronts keep the pair in one (the caller's x mod 64
+        // condition); apply_pre -1: the caller's list has no pair apart
+        if (L.nx % 64u != 0 && apply_pre > 0) {
             if (even) hipLaunchKernelGGL((k_bc_pressure_edge<S, true>), edge, b, 0, st, L, gp);
             else hipLaunchKernelGGL((k_bc_pressure_edge<S, false>), edge, b, 0, st, L, gp);
         }

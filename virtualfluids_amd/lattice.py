@@ -320,9 +320,10 @@ class Lattice:
         ps = [g.struct(real) for g in post]
         arr = (V.VfxFusedBC * len(ps))(*ps) if ps else None
         pr = pre.struct(real) if pre is not None else None
+        apply = 0 if not apply_pre else 1 if pre is not None and pre.edge else -1
         V.check(V.lib().vfx_k17_step_fused(C.byref(s), int(bool(even)), arr, len(ps),
                                            C.byref(pr) if pr is not None else None, _ptr(any_mask),
-                                           int(bool(apply_pre)), _stream(stream)), "vfx_k17_step_fused")
+                                           apply, _stream(stream)), "vfx_k17_step_fused")
 
     def read_populations(self, even=True, stream=None) -> torch.Tensor:
         out = torch.zeros(self.n_nodes, 27, dtype=torch.float64, device=self.device)
@@ -738,6 +739,9 @@ class FusedGroup:
         base[1:] = np.cumsum(np.bincount(words, minlength=nw))[:-1]
         self.bc = bc
         self.n_nodes = n_nodes
+        # a pressure entry whose neighbour is not in its own 64 consecutive node
+        # numbers: the step needs the launch before it that takes such entries
+        self.edge = bool(np.any(nodes & 63 == (0 if bc.normal == 1 else 63)))
         self.node_mask = torch.from_numpy(mask.view(np.int32)).to(bc.device)
         self.word_base = torch.from_numpy(base.view(np.int32)).to(bc.device)
         self._keep = None

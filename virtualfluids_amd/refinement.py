@@ -491,7 +491,7 @@ class RefinedStepper:
         """Kernel launches of one coarse step in the current schedule."""
         if self._plan_c is not None:
             p = self._plan_c
-            edge = int(self.coarse.dims[0] % 64 != 0)  # outlet nodes whose neighbour is in another wavefront
+            edge = int(self.coarse.dims[0] % 64 != 0 and p.pre.edge)
             return 2 * (1 + len(self.fine_bcs)) + 1 + edge + len(p.residual_post) + len(p.residual_pre) + \
                 (1 if self._one_interface else 2)
         if self.merged:
