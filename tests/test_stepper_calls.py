@@ -1,0 +1,120 @@
+"""Which calls a Stepper makes: a lattice or boundary that replaces a launch is
+stepped through its own, every step, and a precursor's reader may change the
+lattice between steps.  No GPU: the library is a recorder."""
+import numpy as np
+import pytest
+
+import virtualfluids_amd as vfx
+from virtualfluids_amd import _lib, lattice
+
+DIMS = (6, 5, 4)
+LAUNCHES = ("collide_stream", "apply_bc", "turbulent_viscosity_amd")
+
+
+class Library:
+    """Stands in for libvfx: notes each call's name, parity and the lattice's omega."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def call(lat, *args):
+            self.calls.append((name, lat._obj.omega))
+            return 0
+        return call
+
+
+@pytest.fixture
+def library(monkeypatch):
+    lib = Library()
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    monkeypatch.setattr(lattice, "_stream", lambda stream: stream)
+    return lib
+
+
+def _bounce():
+    return vfx.BoundaryCondition(0, [7, 8], np.full((27, 2), 0.5), device="cpu")
+
+
+def _outlet():
+    return vfx.BoundaryCondition(4, [10], rho=[0.0], neighbors=[9], normal=1, device="cpu")
+
+
+def _expected(model):
+    step = ["collide_stream", "apply_bc"] + (["turbulent_viscosity_amd"] if model == "amd" else []) + ["apply_bc"]
+    return step * 3
+
+
+@pytest.mark.parametrize("model", ["none", "amd"])
+@pytest.mark.parametrize("where", ["subclass", "instance", "class"])
+def test_a_replaced_launch_is_called(library, monkeypatch, where, model):
+    seen = []
+
+    def noting(name):
+        original = getattr(vfx.Lattice, name)
+
+        def method(*args, **kw):
+            seen.append(name)
+            return original(*args, **kw)
+        return method
+
+    new = {n: noting(n) for n in LAUNCHES}
+    cls = type("Noting", (vfx.Lattice,), new) if where == "subclass" else vfx.Lattice
+    if where == "class":
+        for n in LAUNCHES:
+            monkeypatch.setattr(vfx.Lattice, n, new[n])
+    lat = cls(DIMS, storage="fp32", omega=1.5, device="cpu", turbulence=model, sgs_constant=0.1)
+    if where == "instance":
+        for n in LAUNCHES:
+            setattr(lat, n, new[n].__get__(lat))
+    vfx.Stepper(lat, "k17", [_bounce(), _outlet()]).step(3)
+    assert seen == _expected(model)
+    assert len(library.calls) == len(seen)
+
+
+def test_a_boundary_with_its_own_tables_makes_them_every_step(library):
+    class Pulsating(vfx.BoundaryCondition):
+        made = 0
+
+        def struct(self, real):
+            self.made += 1
+            return super().struct(real)
+
+    bc = Pulsating(0, [7, 8], np.full((27, 2), 0.5), device="cpu")
+    vfx.Stepper(vfx.Lattice(DIMS, storage="fp32", omega=1.5, device="cpu"), "k17", [bc]).step(4)
+    assert bc.made == 4
+
+
+def test_a_reader_may_change_the_lattice(library):
+    lat = vfx.Lattice(DIMS, storage="fp32", omega=1.5, device="cpu")
+
+    def reader(time):
+        lat.omega += 0.01
+        return np.zeros((3, 2))
+
+    planes = vfx.PrecursorPlanes(np.zeros((4, 1), int), np.full((4, 1), 0.25), 2, 3, reader=reader, device="cpu",
+                                 real=lat._macro_dtype())
+    lat.omega = 1.5
+    bc = vfx.BoundaryCondition(12, [7], np.full((27, 1), 0.5), precursor=planes, device="cpu")
+    vfx.Stepper(lat, "k17", [_bounce(), bc]).step(4)
+    omegas = [o for name, o in library.calls if name == "vfx_collide_stream"]
+    # planes are read from the first time step on: each step's collision sees what the reads before it left
+    assert omegas == pytest.approx([1.5, 1.51, 1.52, 1.53])
+
+
+def test_plain_lattices_make_one_view(library, monkeypatch):
+    lat = vfx.Lattice(DIMS, storage="fp32", omega=1.5, device="cpu")
+    made = []
+    b = _bounce()
+    b.tables(lat._macro_dtype())
+    original = vfx.Lattice.struct
+
+    def struct(self):
+        made.append(1)
+        return original(self)
+
+    monkeypatch.setattr(vfx.Lattice, "struct", struct)
+    monkeypatch.setitem(lattice._LATTICE_LAUNCHES, "struct", struct)
+    vfx.Stepper(lat, "k17", [b]).step(5)
+    assert len(made) == 1
+    assert [n for n, _ in library.calls] == ["vfx_collide_stream", "vfx_bc_apply"] * 5

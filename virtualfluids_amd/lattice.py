@@ -936,6 +936,18 @@ class FusedPlan:
         return FusedPlan(post, pre, residual_post, residual_pre, any_mask)
 
 
+# The launches of a lattice and the tables of a boundary as this module defines
+# them: the time step may hand their views over once for several steps.  Where a
+# subclass, an instance or a patch of the class puts its own in place, every step
+# goes through it.
+_LATTICE_LAUNCHES = {n: Lattice.__dict__[n] for n in ("struct", "collide_stream", "apply_bc", "turbulent_viscosity_amd")}
+_BC_TABLES = {n: BoundaryCondition.__dict__[n] for n in ("struct", "tables")}
+
+
+def _as_defined(obj, methods) -> bool:
+    return all(getattr(type(obj), n, None) is f and n not in getattr(obj, "__dict__", ()) for n, f in methods.items())
+
+
 @dataclass
 class Stepper:
     """The per-level time step of UpdateGrid27::updateGrid without refinement
@@ -987,18 +999,25 @@ class Stepper:
                     self.lattice.apply_bc(bc, self.even, stream=stream)
         self._primed = True
 
+    def _one_view(self) -> bool:
+        """One view of the lattice serves all steps of a call: not where the
+        lattice replaces a launch, nor where a precursor's reader, which the
+        steps call, may change the lattice."""
+        return _as_defined(self.lattice, _LATTICE_LAUNCHES) and \
+            not any(b.precursor is not None and b.precursor.reader is not None for b in self.bcs)
+
     def _bc_call(self, bc, s, stream):
         """bc's launch as a function of the parity, for the steps of one call:
-        the tables are handed over once (lattice view s).  Precursor planes
-        rotate, so those make a new view every step."""
+        the tables are handed over once (lattice view s; None: every step).
+        Precursor planes rotate, so those make a new view every step."""
         lat = self.lattice
-        lat._check_bc(bc)
-        if bc.precursor is not None:
-            def precursor(even):
-                if bc.precursor.reader is not None:
+        if s is None or bc.precursor is not None or not _as_defined(bc, _BC_TABLES):
+            def every_step(even):
+                if bc.precursor is not None and bc.precursor.reader is not None:
                     bc.precursor.advance(self.t, stream)
                 lat.apply_bc(bc, even, stream=stream)
-            return precursor
+            return every_step
+        lat._check_bc(bc)
         b = bc.struct(lat._macro_dtype())
         apply, st = V.lib().vfx_bc_apply, _stream(stream)
         args = C.byref(s), C.byref(b)
@@ -1010,7 +1029,7 @@ class Stepper:
         self._prime(stream)
         if n <= 0:
             return
-        s = lat.struct()
+        s = lat.struct() if self._one_view() else None
         post = [self._bc_call(bc, s, stream) for bc in plan.residual_post]
         pre = [self._bc_call(bc, s, stream) for bc in plan.residual_pre]
         for i in range(n):
@@ -1037,24 +1056,39 @@ class Stepper:
         lat = self.lattice
         # wall models sample the velocities the collision writes
         write_macro = any(getattr(b, "wm", None) is not None for b in self.bcs)
-        tmpl = lat._template(write_macro, self.apply_body_force)
         # the lattice and its tables are handed over once per call, not once per
         # launch: a small lattice's step takes less time than making the views
-        s = lat.struct()
+        s = None
+        if self._one_view():
+            tmpl = lat._template(write_macro, self.apply_body_force)  # makes the arrays the view holds
+            s = lat.struct()
         # precursor inflows run last among the post-collision conditions (UpdateGrid27.cpp:252)
         order = sorted(self.bcs, key=lambda b: b.kind in BoundaryCondition.PRECURSOR)
         post = [self._bc_call(b, s, stream) for b in order if not b.pre_collision]
         pre = [self._bc_call(b, s, stream) for b in self.bcs if b.pre_collision]
-        L, st, view, coll = V.lib(), _stream(stream), C.byref(s), COLLISION[self.collision]
-        amd = self.collision == "k17" and getattr(lat, "turbulence", "none") == "amd"
+        if s is None:
+            def collide(even):
+                lat.collide_stream(self.collision, even, write_macro=write_macro, stream=stream,
+                                   apply_body_force=self.apply_body_force)
+
+            def viscosity():
+                lat.turbulent_viscosity_amd(stream=stream)
+        else:
+            L, st, view, coll = V.lib(), _stream(stream), C.byref(s), COLLISION[self.collision]
+
+            def collide(even):
+                V.check(L.vfx_collide_stream(view, coll, int(even), tmpl, st), "vfx_collide_stream")
+
+            def viscosity():
+                V.check(L.vfx_turbulent_viscosity_amd(view, st), "vfx_turbulent_viscosity_amd")
         for _ in range(n):
-            V.check(L.vfx_collide_stream(view, coll, int(self.even), tmpl, st), "vfx_collide_stream")
+            collide(self.even)
             for run in post:
                 run(self.even)
             self.t += 1
             self.even = not self.even
-            if amd:
-                V.check(L.vfx_turbulent_viscosity_amd(view, st), "vfx_turbulent_viscosity_amd")
+            if self.collision == "k17" and getattr(lat, "turbulence", "none") == "amd":
+                viscosity()
             for run in pre:
                 run(self.even)
 
