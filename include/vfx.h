@@ -147,8 +147,9 @@ typedef struct vfx_lattice {
      * step's workgroups are 256 work items: 0 or 256) and the XCD tile run
      * (workgroups reach the 8 XCDs round robin; consecutive tiles are handed
      * to each XCD in runs of this many, a power of two up to 4096, 1 = plain
-     * order; 0 = the built-in choice: structured step 4 for 2-byte
-     * populations, else 16; sparse step 16, 256 for 8-byte populations).
+     * order; 0 = the built-in choice: structured step 16, but 4 for 2-byte
+     * populations from 2^23 nodes and 256 for 8-byte ones from 2^24 nodes with
+     * dims[0] a multiple of 64; sparse step 16, 256 for 8-byte populations).
      * vfx_k17_autotune measures them.  Other kernels ignore both. */
     uint32_t tile_nodes;
     uint32_t xcd_run;

@@ -43,6 +43,24 @@ def test_every_launch_shape_gives_the_same_bytes(cuda, storage):
             assert same, (tile, run)
 
 
+@pytest.mark.parametrize("storage,dims", [("fp16", (256, 256, 128)), ("fp16", (255, 256, 128)), ("fp64", (256, 256, 256)),
+                                          ("fp64", (256, 256, 255)), ("fp64", (260, 256, 256))])
+def test_built_in_runs_give_the_same_bytes(cuda, storage, dims):
+    """The sizes on both sides of the built-in rule, against the plain block order."""
+    print(f"[built-in run {storage} {dims}]", flush=True)
+    out = []
+    for run in (0, 1):
+        lat = vfx.Lattice(dims, storage=storage, omega=1.8)
+        g = torch.Generator(device="cuda").manual_seed(1)
+        flow = [0.02 * (torch.rand(lat.n_nodes, device="cuda", dtype=torch.float64, generator=g) - 0.5) for _ in range(4)]
+        lat.init_equilibrium(*flow)
+        lat.xcd_run = run
+        for i in range(2):
+            lat.collide_stream("k17", i % 2 == 0)
+        out.append(lat.f)
+    assert torch.equal(*out)
+
+
 def test_autotune_keeps_parity_and_picks_a_shape(cuda):
     print("[k17 autotune fp16]", flush=True)
     a, b = _lattice("fp16"), _lattice("fp16")

@@ -149,7 +149,7 @@ struct Lat {
     void* bf[3];           // per-node body force (T), ApplyBodyForce
     double gforce[3];      // global force, unscaled
     double force_factor;
-    uint32_t xrun_lg;      // 1 + log2 of the XCD tile run of the direct step (0: xcd_run<S>())
+    uint32_t xrun_lg;      // 1 + log2 of the step's XCD tile run (0: built-in, step_run or xcd_run)
     uint32_t tile;         // nodes per workgroup of the direct step (0: built-in)
     const uint4* rgroups;  // sparse: per 64 work items {base node, y stride, z stride, regular}, or NULL
 };
@@ -361,8 +361,7 @@ template <typename T> __device__ __forceinline__ void write_macro(const Lat& L, 
 // order).  Shared lines inside a run meet in one L2.  Runs much longer than
 // this spread the XCDs over distant parts of each plane at once, which costs
 // more than it saves for the 2-byte form.  xcd_run is the built-in run of the
-// row-mapped and sparse steps (k_step_fused, k_step_sparse), step_run that of
-// the structured step, whose tiles are consecutive node numbers.
+// sparse step, step_run that of the structured one.
 constexpr uint32_t kXcds = 8;
 __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t G, uint32_t C)
 {
@@ -370,11 +369,6 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t G, uint32_t C
     return b >= full ? b : (b / span) * span + (b % kXcds) * C + (b / kXcds) % C;
 }
 template <typename S> constexpr uint32_t xcd_run() { return sizeof(S) == 8 ? 256u : 16u; }
-// us per K17 step by run of 4 / 16 / 256 tiles of the built-in width (MI355X):
-// FP16 512x256x256 709 / 733 / 784, 230x171x125 96.1 / 98.8 / 97.6; FP32
-// 512x256x256 1360 / 1359 / 1437; FP64 256^3 1411 / 1434 / 1434, BGK 160^3
-// 362 / 348 / 357
-template <typename S> constexpr uint32_t step_run() { return sizeof(S) == 2 ? 4u : 16u; }
 // the same for a run of 2^lg tiles (shifts only)
 __device__ __forceinline__ uint32_t xcd_block_pow2(uint32_t b, uint32_t G, uint32_t lg)
 {
@@ -401,7 +395,7 @@ __device__ __forceinline__ void step_direct_body(const Lat& L, const Rates<typen
                                                  uint32_t blocks)
 {
     using T = typename Compute<S>::T;
-    const uint32_t blk = L.xrun_lg ? xcd_block_pow2(block, blocks, L.xrun_lg - 1u) : xcd_block(block, blocks, step_run<S>());
+    const uint32_t blk = xcd_block_pow2(block, blocks, L.xrun_lg - 1u);
     const uint32_t k = blk * blockDim.x + threadIdx.x;
     if (k >= (uint32_t)L.N) return;
     uint32_t kk[8];
@@ -1951,8 +1945,7 @@ __global__ void __launch_bounds__(256) k_step_pre(Lat L, Rates<typename Compute<
     using T = typename Compute<S>::T;
     constexpr bool FAST = sizeof(S) != 8;
     constexpr bool O2 = sizeof(S) == 2;
-    const uint32_t blk = L.xrun_lg ? xcd_block_pow2(blockIdx.x, gridDim.x, L.xrun_lg - 1u)
-                                   : xcd_block(blockIdx.x, gridDim.x, step_run<S>());
+    const uint32_t blk = xcd_block_pow2(blockIdx.x, gridDim.x, L.xrun_lg - 1u);
     const uint32_t k = blk * blockDim.x + threadIdx.x;
     const bool active = k < (uint32_t)L.N && !is_solid(L, k);
     // the group's words are read before the populations, so that a boundary
@@ -2345,13 +2338,42 @@ template <typename S, int COLL, bool FAST> constexpr unsigned step_lds_cap()
                : 0u;
 }
 
+// Built-in XCD run of the structured step, by where the 54 streams' lines are
+// when they are needed again.  Boxes that mostly stay in the 256 MiB last-level
+// cache and all FP32 ones: 16.  FP16 from 2^23 nodes: 4.  FP64 from 2^24 nodes
+// with rows of whole lines (planes and rows on the same few channels): 256, so
+// that an XCD stays in its own pages.  MI355X, us per K17 step by run of 4 / 16 /
+// 64 / 256 tiles of the built-in width, the rule's lines lie between:
+//   FP16 128^3 53 / 43 / 43 / 43, 256x128x128 97 / 81 / 81, 160^3 83 / 82 / 81,
+//     192^3 151 / 149 / 150 | 256x256x128 181 / 185, 224^3 248 / 250,
+//     320x256x160 285 / 287, 384x256x256 528 / 534, 512x256x256 707 / 727 / 726 /
+//     780, 512^3 2840 / 2921 / 2950
+//   FP32 128^3 67 / 69, 160^3 180 / 176, 256x256x64 190 / 181, 256^3 657 / 670 /
+//     674 / 717, 333x301x290 1263 / 1249 / 1243
+//   FP64 160^3 372 / 357 / 359 / 369, 256x256x128 714 / 716 / 732 / 720,
+//     301x257x203 1418 / 1367 / 1369 / 1379, 333^3 3550 / 3226 / 3233 / 3261 |
+//     256^3 1414 / 1436 / 1449 / 1429, 512x256x256 2924 / 2921 / 2887 / 2806 (BGK
+//     2905 / 2902 / 2869 / 2841), 512x512x128 2879 / 2867 / 2841 / 2815,
+//     640x384x150 3363 / 3177 / 3187 / 3151
+template <typename S> inline uint32_t step_run(const Lat& L)
+{
+    if (sizeof(S) == 2) return L.N >= (1u << 23) ? 4u : 16u;
+    return sizeof(S) == 8 && L.N >= (1u << 24) && L.nx % 64u == 0 ? 256u : 16u;
+}
+template <typename S> inline Lat with_run(const Lat& in)
+{
+    Lat L = in;
+    if (!L.xrun_lg) L.xrun_lg = 1u + (uint32_t)__builtin_ctz(step_run<S>(in));
+    return L;
+}
+
 template <typename S, int COLL, bool EVEN, bool FAST>
 hipError_t launch_step_t(const Lat& L, int direct, const Rates<typename Compute<S>::T>& R, hipStream_t st)
 {
     if (direct) {
         const unsigned tile = L.tile ? L.tile : step_lds_cap<S, COLL, FAST>() ? 128u : 256u;
         hipLaunchKernelGGL((k_step_direct<S, COLL, EVEN, FAST>), dim3(grid_for(L.N, tile)), dim3(tile),
-                           (step_lds_cap<S, COLL, FAST>()), st, L, R);
+                           (step_lds_cap<S, COLL, FAST>()), st, with_run<S>(L), R);
     } else {
         const uint64_t n = node_items(L, 0);
         if (n == 0) return hipSuccess;
@@ -2441,8 +2463,8 @@ hipError_t launch_step_fused(const Lat& L, bool even, double omega, const double
         const unsigned tile = L.tile ? L.tile : sizeof(S) == 4 ? 128u : 256u;
         const dim3 g(grid_for(L.N, tile)), t(tile);
         constexpr unsigned lds = step_lds_cap<S, VFX_K17, sizeof(S) != 8>();
-        if (even) hipLaunchKernelGGL((k_step_pre<S, true>), g, t, lds, st, L, R, gp);
-        else hipLaunchKernelGGL((k_step_pre<S, false>), g, t, lds, st, L, R, gp);
+        if (even) hipLaunchKernelGGL((k_step_pre<S, true>), g, t, lds, st, with_run<S>(L), R, gp);
+        else hipLaunchKernelGGL((k_step_pre<S, false>), g, t, lds, st, with_run<S>(L), R, gp);
         e = hipGetLastError();
     } else {
         constexpr bool FAST = sizeof(S) != 8;
@@ -2490,7 +2512,7 @@ template <typename S> hipError_t launch_step_levels(const LevelInput* in, int n,
     const uint32_t tile = in[0].L.tile == in[1].L.tile && in[0].L.tile ? in[0].L.tile : 256u;
     uint32_t first = 0;
     for (int j = 0; j < n; ++j) {
-        *L[j] = in[j].L;
+        *L[j] = with_run<S>(in[j].L);
         *R[j] = make_rates<T>(in[j].omega, in[j].lim, in[j].force, 0.0);
         *blocks[j] = grid_for(L[j]->N, tile);
         if (j == 1) P.first1 = first;
