@@ -427,8 +427,7 @@ def channel_leg(torch, vfx, steps, sample_every=10, forms=("fp64", "fp32", "fp16
     every `sample_every` steps.  The pressure outlet runs inside the
     collide-stream kernel (Stepper(fuse=True, fuse_post=False)), the
     interpolated groups as kernels of their own; `separate_steps` FP16 steps
-    with every group separate, and with every group fused, are timed beside
-    it.  Reports
+    with every group separate are timed beside it.  Reports
     whole-step MLUPS (fluid nodes, all boundary kernels and statistics
     included), the time-averaged mean velocity error of FP32/FP16 storage vs
     FP64, and the FP64 mass/momentum monitor."""
@@ -471,8 +470,8 @@ def channel_leg(torch, vfx, steps, sample_every=10, forms=("fp64", "fp32", "fp16
              "separate_kernels": len(plan.residual_post) + len(plan.residual_pre)}
         if storage == "fp16" and separate_steps > 0:
             # the leg's own policy without the statistics, the same channel
-            # with one kernel per boundary group, and with every group inside
-            # the collide-stream kernel
+            # with one kernel per boundary group, and with the default
+            # fuse_post (the same steps as the first)
             n_sep = separate_steps // 10 * 10
             for name, kw in (("pressure_fused_without_statistics", {"fuse": True, "fuse_post": False}),
                              ("separate_bc_kernels", {}), ("all_groups_fused", {"fuse": True})):

@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 
 import virtualfluids_amd as vfx
-from virtualfluids_amd import _lib, lattice
+from tests.test_geometry import small_channel
+from virtualfluids_amd import _lib, geometry, lattice
 
 DIMS = (6, 5, 4)
 LAUNCHES = ("collide_stream", "apply_bc", "turbulent_viscosity_amd")
@@ -118,3 +119,35 @@ def test_plain_lattices_make_one_view(library, monkeypatch):
     vfx.Stepper(lat, "k17", [b]).step(5)
     assert len(made) == 1
     assert [n for n, _ in library.calls] == ["vfx_collide_stream", "vfx_bc_apply"] * 5
+
+
+@pytest.mark.parametrize("fuse_post", [True, False])
+def test_fused_steps_run_other_boundaries_whole(library, fuse_post):
+    """One launch per boundary that is not inside the step, in the listed order,
+    also where only some of its entries could be a group of the step's call."""
+    ch = small_channel()
+    solid = ch.solid.copy()
+    wall = next(t for t in ch.bcs if t.kind == 1)
+    k, d = int(wall.nodes[0]), int(np.flatnonzero(wall.q27[:, 0] >= 0)[0])
+    nx, ny, nz = ch.dims
+    x, y, z = (k % nx + vfx.CX[d]) % nx, (k // nx % ny + vfx.CY[d]) % ny, (k // (nx * ny) + vfx.CZ[d]) % nz
+    solid[x + nx * (y + ny * z)] = False  # this entry's link ends in a fluid node
+    seen = []
+
+    class Noting(vfx.Lattice):
+        def k17_step_fused(self, even, post=(), pre=None, apply_pre=False, any_mask=None, stream=None):
+            seen.append((list(post), pre is not None, any_mask))
+
+        def apply_bc(self, bc, even=True, stream=None):
+            seen.append(bc)
+
+    bcs = geometry.boundary_conditions(ch.bcs, device="cpu")
+    st = vfx.Stepper(Noting(ch.dims, storage="fp32", omega=1.5, solid=solid, device="cpu"), "k17", bcs, fuse=True,
+                     fuse_post=fuse_post)
+    assert vfx.FusedPlan.build(st.lattice, bcs).residual_post
+    st.step(2)
+    post = [b for b in bcs if not b.pre_collision]
+    assert len(post) == 2
+    outlet = seen.pop()
+    assert outlet.kind == 4 and outlet.n == next(b for b in bcs if b.pre_collision).n
+    assert seen == [([], True, None)] + post + [([], True, None)] + post

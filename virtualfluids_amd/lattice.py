@@ -311,7 +311,7 @@ class Lattice:
         (vfx_k17_step_fused): up to two post-collision FusedGroups and one
         pressure FusedGroup whose values the step takes from the previous
         step's populations (apply_pre False on the first step of a run);
-        any_mask: the union of the groups' node masks (FusedPlan.any_mask)."""
+        any_mask: the union of the groups' node masks (not read)."""
         real = self._macro_dtype()
         for g in list(post) + ([pre] if pre is not None else []):
             if g.bc.max_node >= self.n_nodes or g.n_nodes != self.n_nodes:
@@ -722,8 +722,7 @@ FUSED_POST_KINDS = (V.VFX_BC_NOSLIP_INTERPOLATED, V.VFX_BC_VELOCITY_INTERPOLATED
 
 
 class FusedGroup:
-    """A boundary whose entries the collide-stream kernel applies itself
-    (vfx_fused_bc): entries sorted by node, one per node; node_mask has bit k
+    """A boundary taken along with a step (vfx_fused_bc): entries sorted by node, one per node; node_mask has bit k
     set for every node k of the group, word_base[w] counts the entries of the
     nodes below 32 w."""
 
@@ -768,8 +767,8 @@ def _unique_nodes(nodes) -> np.ndarray:
 
 
 def fusable_post_entries(lattice, bc) -> np.ndarray:
-    """Entries of an interpolated boundary the collide-stream kernel may apply
-    itself: the node is fluid, appears once, and the far node of every wall
+    """Entries of an interpolated boundary that may be a post group of
+    vfx_k17_step_fused: the node is fluid, appears once, and the far node of every wall
     link (0 <= q <= 1, in the storage real's rounding too) is solid, so that no
     other thread of the launch touches the elements the boundary writes or
     the node's own post-collision elements it reads back."""
@@ -875,21 +874,21 @@ def step_levels(levels, stream=None):
 
 @dataclass
 class FusedPlan:
-    """Which boundary entries a fused step takes along (post: up to two groups,
-    pre: one pressure group, inside the collide-stream kernel) and which run as
-    boundary kernels of their own (residual_post / residual_pre, in the order
-    of the unfused step)."""
+    """Which boundary entries one Lattice.k17_step_fused call may take along
+    (post: up to two groups, run by their own kernels after the step; pre: one
+    pressure group, inside the collide-stream kernel) and which are left to
+    apply_bc (residual_post / residual_pre, in the order of the unfused step)."""
 
     post: list
     pre: FusedGroup | None
     residual_post: list
     residual_pre: list
-    any_mask: torch.Tensor | None = None  # union of the groups' node masks
+    any_mask: torch.Tensor | None = None  # union of the groups' node masks (the library does not read it)
 
     @staticmethod
     def build(lattice, bcs, post=True) -> "FusedPlan":
-        """post=False: only the pressure group is fused (the interpolated
-        kinds run as separate kernels)."""
+        """post=False: only the pressure group is taken along (the interpolated
+        kinds stay whole in residual_post)."""
         def split(b, ok):
             sel = np.flatnonzero(ok)
             sel = sel[np.argsort(b.nodes[sel], kind="stable")]
@@ -929,10 +928,9 @@ class FusedPlan:
         groups = post + ([pre] if pre is not None else [])
         any_mask = None
         if groups:
-            u = groups[0].node_mask.clone()
+            any_mask = groups[0].node_mask
             for g in groups[1:]:
-                u |= g.node_mask
-            any_mask = u
+                any_mask = any_mask | g.node_mask
         return FusedPlan(post, pre, residual_post, residual_pre, any_mask)
 
 
@@ -962,12 +960,12 @@ class Stepper:
     even: bool = True
     apply_body_force: bool = False  # CollisionTemplate ApplyBodyForce (Lattice.set_body_force)
     t: int = 1  # time step of the next step; precursor planes with a reader cycle on it
-    # Apply the interpolated and pressure boundaries inside the collide-stream
-    # kernel where the geometry allows (FusedPlan); same populations as the
-    # separate boundary kernels.
+    # Apply the pressure boundary inside the collide-stream kernel where the
+    # geometry allows (FusedPlan); same populations as the separate boundary
+    # kernels, which the other boundaries run as, each whole.
     fuse: bool = False
-    # with fuse: also the interpolated kinds are part of the step's call (False:
-    # the pressure group only); they run as kernels of their own either way
+    # whether fused_plan() also groups the interpolated kinds, for callers that
+    # hand them to Lattice.k17_step_fused themselves; the steps are the same
     fuse_post: bool = True
     # Before the first step, apply the non-reflecting outflow kinds once with
     # the starting parity: they write the populations the step after next
@@ -975,10 +973,13 @@ class Stepper:
     # held (False leaves that to the caller, as VirtualFluids does).
     prime_outflow: bool = True
     _primed: bool = field(default=False, init=False, repr=False)
-    _plan: FusedPlan | None = field(default=None, init=False, repr=False)
+    _plans: dict = field(default_factory=dict, init=False, repr=False)
     _plan_key: tuple | None = field(default=None, init=False, repr=False)
 
     def fused_plan(self) -> FusedPlan:
+        return self._plan(self.fuse_post)
+
+    def _plan(self, post) -> FusedPlan:
         lat = self.lattice
         if not lat.direct or self.collision != "k17" or lat.variant != "default" or \
                 getattr(lat, "turbulence", "none") != "none" or self.apply_body_force:
@@ -986,11 +987,12 @@ class Stepper:
                              "without turbulence model or body-force arrays")
         if any(getattr(b, "wm", None) is not None for b in self.bcs):
             raise ValueError("fused boundaries do not run with wall models")
-        key = (id(lat), tuple(id(b) for b in self.bcs), self.fuse_post)
+        key = (id(lat), tuple(id(b) for b in self.bcs))
         if self._plan_key != key:
-            self._plan = FusedPlan.build(lat, self.bcs, post=self.fuse_post)
-            self._plan_key = key
-        return self._plan
+            self._plans, self._plan_key = {}, key
+        if post not in self._plans:
+            self._plans[post] = FusedPlan.build(lat, self.bcs, post=post)
+        return self._plans[post]
 
     def _prime(self, stream):
         if self.prime_outflow and not self._primed:
@@ -1024,7 +1026,7 @@ class Stepper:
         return lambda even: V.check(apply(*args, int(even), st), "vfx_bc_apply")
 
     def _step_fused(self, n, stream):
-        plan = self.fused_plan()
+        plan = self._plan(False)  # the pressure group; the other boundaries whole
         lat = self.lattice
         self._prime(stream)
         if n <= 0:
@@ -1035,8 +1037,7 @@ class Stepper:
         for i in range(n):
             # the pressure group of the previous step of this run is applied
             # while the node's populations are gathered
-            lat.k17_step_fused(self.even, plan.post, plan.pre, apply_pre=i > 0, any_mask=plan.any_mask,
-                               stream=stream)
+            lat.k17_step_fused(self.even, (), plan.pre, apply_pre=i > 0, stream=stream)
             for run in post:
                 run(self.even)
             self.t += 1

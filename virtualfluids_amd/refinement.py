@@ -429,7 +429,7 @@ class RefinedStepper:
 
     def _coarse_step_fused(self, even, first, stream):
         plan, lat = self._plan_c, self.coarse
-        lat.k17_step_fused(even, [], plan.pre, apply_pre=not first, any_mask=plan.any_mask, stream=stream)
+        lat.k17_step_fused(even, [], plan.pre, apply_pre=not first, stream=stream)
         for bc in plan.residual_post:
             lat.apply_bc(bc, even, stream=stream)
         for bc in plan.residual_pre:
