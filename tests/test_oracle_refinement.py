@@ -384,3 +384,23 @@ def test_interface_cells_apart_on_the_nests():
     bad = copy.copy(nest)
     bad.fc_coarse = np.concatenate([nest.fc_coarse, _cell_corners(nest.cf_coarse[:1], nest.coarse_dims)[:1]])
     assert not interface_cells_apart(bad)
+
+
+@pytest.mark.parametrize("merged", [False, True])
+@pytest.mark.parametrize("field", ["fc_coarse", "fc_fine", "cf_coarse", "cf_fine"])
+def test_interface_cells_beyond_a_level_are_refused(field, merged):
+    """A ValueError, as scale_fc and scale_cf raise it, whatever the schedule."""
+    nest = vfx.NestedBox((12, 12, 12), (2, 2, 2), (9, 9, 9))
+    cells = getattr(nest, field).copy()
+    cells[0] = 10 ** 6
+    setattr(nest, field, cells)
+    with pytest.raises(ValueError, match="beyond its lattice"):
+        vfx.RefinedStepper(nest, 1.5, storage="fp32", device="cpu", merged=merged)
+
+
+def test_interface_without_cells():
+    """Cell lists given as empty lists: nothing meets, the levels step apart."""
+    nest = vfx.NestedBox((12, 12, 12), (2, 2, 2), (9, 9, 9))
+    for field in ("fc_coarse", "fc_fine", "cf_coarse", "cf_fine"):
+        setattr(nest, field, [])
+    assert vfx.RefinedStepper(nest, 1.5, storage="fp32", device="cpu").fc.n == 0

@@ -278,7 +278,7 @@ def interface_cells_apart(nest) -> bool:
             m[k] = True
         return m
 
-    coarse = marked([np.asarray(nest.fc_coarse)], nest.coarse_dims)
+    coarse = marked([np.asarray(nest.fc_coarse, dtype=np.int64)], nest.coarse_dims)
     if any(coarse[k].any() for k in _corners(nest.cf_coarse, nest.coarse_dims)):
         return False
     fine = marked(_corners(nest.cf_fine, nest.fine_dims), nest.fine_dims)
@@ -332,6 +332,8 @@ class RefinedStepper:
             bc.tables(real)
         self.fc.offsets(real)
         self.cf.offsets(real)
+        for cells in (self.fc, self.cf):
+            _check_cells(self.coarse, self.fine, cells)
         # both interface interpolations in one launch where the nest keeps them
         # apart: each alone is bound by latency and by the cache lines of the
         # faces normal to x
