@@ -82,6 +82,23 @@ def test_invalid_arguments_fail_without_device():
     assert L.vfx_version() >= 1
 
 
+def test_box_whose_node_count_exceeds_64_bits_is_refused():
+    """dims whose product is n_nodes modulo 2^64 only: (2^34 + 1) 2^30 = 2^64 + 2^30."""
+    L = vfx.lib()
+    V = vfx._lib
+    s = V.VfxLattice()
+    s.f = 1
+    s.storage = 2
+    s.fp16_scale = 1.0
+    s.omega = 1.5
+    s.direct = 1
+    s.n_nodes = 2 ** 30
+    s.dims[:] = [2 ** 30, 5, (2 ** 34 + 1) // 5]
+    assert s.dims[0] * s.dims[1] * s.dims[2] % 2 ** 64 == s.n_nodes
+    assert L.vfx_collide_stream(C.byref(s), 0, 1, 0, None) == V.VFX_EINVAL
+    assert b"n_nodes" in L.vfx_last_error()
+
+
 def test_refinement_arguments_fail_without_device():
     L = vfx.lib()
     V = vfx._lib

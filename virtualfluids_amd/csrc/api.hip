@@ -70,16 +70,16 @@ vfx_status make_lat(const vfx_lattice* in, vfx::Lat& L)
     if (in->direct) {
         const uint64_t nx = in->dims[0], ny = in->dims[1], nz = in->dims[2];
         if (nx == 0 || ny == 0 || nz == 0) return fail(VFX_EINVAL, "direct addressing needs dims > 0");
-        if (nx * ny * nz != in->n_nodes)
+        if (ny * nz > in->n_nodes / nx || nx * ny * nz != in->n_nodes) // the product may exceed 64 bits
             return fail(VFX_EINVAL, "dims %llu*%llu*%llu != n_nodes %llu", (unsigned long long)nx,
                         (unsigned long long)ny, (unsigned long long)nz, (unsigned long long)in->n_nodes);
-        const uint64_t tile = in->tile_nodes ? in->tile_nodes : 256;
-        if (tile != 64 && tile != 128 && tile != 256) return fail(VFX_EINVAL, "tile_nodes must be 0, 64, 128 or 256");
-        if (ny * nz >= (1ull << 31) / ((nx + tile - 1) / tile)) return fail(VFX_EUNSUPPORTED, "grid too large");
+        const uint32_t tile = in->tile_nodes;
+        if (tile != 0 && tile != 64 && tile != 128 && tile != 256)
+            return fail(VFX_EINVAL, "tile_nodes must be 0, 64, 128 or 256");
         L.nx = (uint32_t)nx;
         L.ny = (uint32_t)ny;
         L.nz = (uint32_t)nz;
-        L.tile = in->tile_nodes;
+        L.tile = tile;
         L.div_x = vfx::make_fastdiv(L.nx);
         L.div_y = vfx::make_fastdiv(L.ny);
         L.solid = in->solid_mask;
