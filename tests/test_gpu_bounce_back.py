@@ -1,4 +1,4 @@
-"""The bounce-back kernel (one thread per link) on lists whose length sits at the
+"""The bounce-back kernel (one thread per pair of links) on lists whose length sits at the
 edges of a wavefront and a workgroup, with links chosen at random: every element
 of the array against the formula, on the structured and the sparse layout, and
 the boundary set's one-thread-per-node form against the kernel bit for bit."""
@@ -15,9 +15,9 @@ DIMS = (16, 16, 18)
 N = int(np.prod(DIMS))
 
 
-def _at(k, d):
+def _at(k, d, dims=DIMS):
     """The node direction d of node k lives on (one step along every axis with c_d < 0, periodic)."""
-    nx, ny, nz = DIMS
+    nx, ny, nz = dims
     x, y, z = k % nx + (CX[d] < 0), k // nx % ny + (CY[d] < 0), k // (nx * ny) + (CZ[d] < 0)
     return x % nx + nx * (y % ny + ny * (z % nz))
 
@@ -66,6 +66,33 @@ def test_links_fp64(cuda, n, sparse, even):
     got = lat.f.cpu().numpy().reshape(27, N)
     # 6 w rounded once here, 4/9, 1/9 and 1/36 in the kernel: one unit in the last place of a wall term <= 0.07
     assert np.abs(got - ref).max() <= 2e-17
+
+
+@pytest.mark.parametrize("sparse", [False, True])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_a_node_that_is_its_own_neighbour(cuda, axis, sparse):
+    """A box one node thick with walls on both sides: a link and its opposite
+    exchange their two populations, as the formula on the array before."""
+    print(f"[bounce back axis {axis} {sparse}]", flush=True)
+    dims = [8, 6, 16]
+    dims[axis] = 1
+    n = int(np.prod(dims))
+    x = np.arange(n) % dims[0], np.arange(n) // dims[0] % dims[1], np.arange(n) // (dims[0] * dims[1])
+    nodes = np.flatnonzero((x[0] % 2 == 0) & (x[1] % 2 == 0) & (x[2] % 2 == 0))
+    f = np.random.default_rng(axis).uniform(-1e-2, 1e-2, 27 * n)
+    if sparse:
+        k = np.arange(n, dtype=np.uint32)
+        lat = vfx.Lattice(storage="fp64", omega=1.7, neighbors=[_at(k, d, dims).astype(np.uint32) for d in (2, 4, 6)],
+                          fluid_nodes=k)
+    else:
+        lat = vfx.Lattice(tuple(dims), storage="fp64", omega=1.7)
+    lat.f.copy_(torch.from_numpy(f))
+    lat.apply_bc(vfx.BoundaryCondition(0, nodes, np.full((27, nodes.size), 0.5)), True)
+    ref = f.reshape(27, n).copy()
+    for d in range(1, 27):
+        at = _at(nodes, INV[d], dims)
+        ref[d, at] = f.reshape(27, n)[INV[d], at]
+    assert np.array_equal(lat.f.cpu().numpy().reshape(27, n), ref)
 
 
 @pytest.mark.parametrize("storage", ["fp64", "fp32", "fp16"])

@@ -1212,21 +1212,23 @@ __device__ __forceinline__ T bb_value(int d, T fpost, T ux, T uy, T uz, int cpu_
     else return fpost - coef * s;
 }
 
-// Links D0 .. D0 + G - 1 (up to 26) of entry i: every fraction is loaded first,
-// then the populations of the wall links, then they are stored
-template <typename S, bool EVEN, int D0, int G>
+// Links DIR of entry i: every fraction is loaded first, then the populations of
+// the wall links, then they are stored
+template <typename S, bool EVEN, int... DIR>
 __device__ __forceinline__ void bb_links(const Lat& L, const BCDev& B, uint32_t i)
 {
     using T = typename Compute<S>::T;
-    constexpr int D1 = D0 + G < 27 ? D0 + G : 27;
+    constexpr int G = sizeof...(DIR);
+    constexpr int dir[G] = {DIR...};
     const uint32_t k = B.k[i];
     bool on[G];
     bool any = false;
 #pragma unroll
-    for (int d = D0; d < D1; ++d) {
+    for (int j = 0; j < G; ++j) {
+        const int d = dir[j];
         const T q = bc_q<T>(B, d, i);
-        on[d - D0] = q >= T(0) && q <= T(1);
-        any |= on[d - D0];
+        on[j] = q >= T(0) && q <= T(1);
+        any |= on[j];
     }
     if (!any || k >= L.N) return; // malformed list entry: never touch memory outside the lattice
     uint32_t kk[8];
@@ -1235,52 +1237,58 @@ __device__ __forceinline__ void bb_links(const Lat& L, const BCDev& B, uint32_t 
     T ux = B.vx ? bc_at<T>(B.vx, i) : T(0), uy = B.vy ? bc_at<T>(B.vy, i) : T(0), uz = B.vz ? bc_at<T>(B.vz, i) : T(0);
     T f[G];
 #pragma unroll
-    for (int d = D0; d < D1; ++d) {
+    for (int j = 0; j < G; ++j) {
+        const int d = dir[j];
         // post-collision population of direction d sits where e was read from
         const int e = inv(d);
-        if (on[d - D0])
-            f[d - D0] = Storage<S, T>::ld(plane<S>(L, slot(e, EVEN)), kk[nbr(e)], L.ld[weight_class(d)], L.sh[d]);
+        if (on[j])
+            f[j] = Storage<S, T>::ld(plane<S>(L, slot(e, EVEN)), kk[nbr(e)], L.ld[weight_class(d)], L.sh[d]);
     }
 #pragma unroll
-    for (int d = D0; d < D1; ++d) {
+    for (int j = 0; j < G; ++j) {
+        const int d = dir[j];
         // next step (parity !EVEN) reads direction e of node k from here
         const int e = inv(d);
-        if (on[d - D0])
-            Storage<S, T>::st(plane<S>(L, slot(e, !EVEN)), kk[nbr(e)], bb_value<T>(d, f[d - D0], ux, uy, uz, B.cpu_float),
+        if (on[j])
+            Storage<S, T>::st(plane<S>(L, slot(e, !EVEN)), kk[nbr(e)], bb_value<T>(d, f[j], ux, uy, uz, B.cpu_float),
                               L.st[weight_class(e)], L.ss[e]);
     }
 }
 template <typename S, bool EVEN>
 __device__ __forceinline__ void bc_velocity_bb_entry(const Lat& L, const BCDev& B, uint32_t i)
 {
-    if (i < B.n) bb_links<S, EVEN, 1, 26>(L, B, i);
+    if (i < B.n)
+        bb_links<S, EVEN, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, 18, 19, 20, 21, 22, 23, 24, 25, 26>(L, B, i);
 }
 
-// One thread per link: blockIdx.y is the direction, so a wavefront holds one
-// direction of 64 boundary nodes and everything about the link is a constant of
-// the switch branch it takes.  Short lists are bound by latency: with the links
-// of a node one after another in one thread each waited for the one before (its
+// One thread per link and its opposite: blockIdx.y is the pair, so a wavefront
+// holds one pair of 64 boundary nodes and everything about its links is a
+// constant of the switch branch it takes.  The two stay in one thread because
+// they exchange the same two elements where a node is its own neighbour along
+// them (an axis of one node): loads first, then stores.  Any other element is
+// touched by one link only.  Lists are bound by latency: with the links of a
+// node one after another in one thread each waited for the one before (its
 // fraction, its population and its store, 26 round trips); here the chain is
-// fraction -> population -> store.  Long lists are bound by the cache lines of
-// faces normal to x, one per element.  MI355X, us per launch, before -> now:
-// cavity 30^3 FP32 13.6 -> 3.6, 64^3 FP64 17.5 -> 6.2, y and z walls and spheres
-// of a 320x130x134 sparse box FP16 33.9 -> 31.0; 3, 7, 13 and 26 links per
-// thread: 30^3 4.3 / 4.7 / 5.8 / 7.3, 128^3 FP16 14.4 / 14.9 / 14.9 / 15.9
-// against 15.9.
+// fraction -> population -> store.  Long sparse lists add the neighbour indices
+// to it (up to three dependent loads) and read every fraction and node number,
+// 27 x 8 bytes a node, for the third of the links that are walls.  MI355X, us
+// per launch: a thread for all links of a node, one after another, against one
+// per link, cavity 30^3 FP32 13.6 and 3.6, 64^3 FP64 17.5 and 6.2; one per link
+// against one per pair, launches back to back, 4.5 and 4.4, 5.9 and 5.5; 4 steps
+// with y and z walls and spheres of a 320x130x134 sparse box, FP16, 673 and 664.
 template <typename S, bool EVEN>
 __global__ void __launch_bounds__(256) k_bc_velocity_bb(Lat L, BCDev B)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= B.n) return;
-#define VFX_LINK(D) \
-    case D: bb_links<S, EVEN, D, 1>(L, B, i); break;
-    switch (blockIdx.y + 1) {
-        VFX_LINK(1) VFX_LINK(2) VFX_LINK(3) VFX_LINK(4) VFX_LINK(5) VFX_LINK(6) VFX_LINK(7) VFX_LINK(8) VFX_LINK(9)
-        VFX_LINK(10) VFX_LINK(11) VFX_LINK(12) VFX_LINK(13) VFX_LINK(14) VFX_LINK(15) VFX_LINK(16) VFX_LINK(17)
-        VFX_LINK(18) VFX_LINK(19) VFX_LINK(20) VFX_LINK(21) VFX_LINK(22) VFX_LINK(23) VFX_LINK(24) VFX_LINK(25)
-        VFX_LINK(26)
+#define VFX_PAIR(Y, D) \
+    case Y: bb_links<S, EVEN, D, inv(D)>(L, B, i); break;
+    switch (blockIdx.y) {
+        VFX_PAIR(0, dP00) VFX_PAIR(1, d0P0) VFX_PAIR(2, d00P) VFX_PAIR(3, dPP0) VFX_PAIR(4, dPM0) VFX_PAIR(5, dP0P)
+        VFX_PAIR(6, dP0M) VFX_PAIR(7, d0PP) VFX_PAIR(8, d0PM) VFX_PAIR(9, dPPP) VFX_PAIR(10, dPPM) VFX_PAIR(11, dPMP)
+        VFX_PAIR(12, dMPP)
     }
-#undef VFX_LINK
+#undef VFX_PAIR
 }
 
 // Interpolated bounce-back family (NoSlipInterpolatedCompressible.cu:44-378,
@@ -2700,8 +2708,8 @@ template <typename S> hipError_t launch_bc(const Lat& L, const BCDev& B, int kin
     const dim3 g(grid_for(B.n, kBlock)), b(kBlock);
     switch (kind) {
     case VFX_BC_VELOCITY_BOUNCE_BACK:
-        if (even) hipLaunchKernelGGL((k_bc_velocity_bb<S, true>), dim3(g.x, 26), b, 0, st, L, B);
-        else hipLaunchKernelGGL((k_bc_velocity_bb<S, false>), dim3(g.x, 26), b, 0, st, L, B);
+        if (even) hipLaunchKernelGGL((k_bc_velocity_bb<S, true>), dim3(g.x, 13), b, 0, st, L, B);
+        else hipLaunchKernelGGL((k_bc_velocity_bb<S, false>), dim3(g.x, 13), b, 0, st, L, B);
         break;
     case VFX_BC_NOSLIP_INTERPOLATED:
         if (even) hipLaunchKernelGGL((k_bc_interp<S, true, VFX_BC_NOSLIP_INTERPOLATED>), g, b, 0, st, L, B);
