@@ -1270,8 +1270,8 @@ __device__ __forceinline__ void bc_velocity_bb_entry(const Lat& L, const BCDev& 
 // node one after another in one thread each waited for the one before (its
 // fraction, its population and its store, 26 round trips); here the chain is
 // fraction -> population -> store.  Long sparse lists add the neighbour indices
-// to it (up to three dependent loads) and read every fraction and node number,
-// 27 x 8 bytes a node, for the third of the links that are walls.  MI355X, us
+// to it (up to three dependent loads) and read 26 fractions and 13 node numbers
+// a node, of which a third are walls.  MI355X, us
 // per launch: a thread for all links of a node, one after another, against one
 // per link, cavity 30^3 FP32 13.6 and 3.6, 64^3 FP64 17.5 and 6.2; one per link
 // against one per pair, launches back to back, 4.5 and 4.4, 5.9 and 5.5; 4 steps
@@ -1939,8 +1939,9 @@ __device__ __forceinline__ void fused_pressure(const Lat& L, const FusedGroup& G
 // in the wavefronts that hold a boundary node, where a kernel of its own reads
 // 27 and writes 18 cache lines per node of the face.  Every lane forms its own
 // density and velocity and the lanes pass one population at a time, so no second
-// set of 27 registers is live (73 VGPRs for FP16, nothing spilled; held to 72
-// the step schedules worse, 190 us); the group's words are read before the
+// set of 27 registers is live (73 VGPRs for FP16 and FP32, 6 wavefronts per SIMD,
+// 122 and 4 for FP64; FP16 keeps 12 to 17 scalars in lanes of a vector register;
+// held to 72 the step schedules worse, 190 us); the group's words are read before the
 // populations, the entry while they arrive (after them: 150 us).  A boundary
 // node whose neighbour is in another wavefront (lane 0, or 63 for -x) is left to
 // k_bc_pressure_edge, launched before where the list has one.  MI355X, us per
