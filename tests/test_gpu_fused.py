@@ -1,9 +1,10 @@
-"""Boundary conditions applied inside the collide-stream kernel
-(vfx_k17_step_fused through Stepper(fuse=True)) against the separate boundary
-kernels of the unfused step: the stored populations agree bit for bit in FP64,
-FP32 and FP16 storage, over runs split into several step() calls, with the
-entries the kernel cannot take left to residual kernels; FP64 also against the
-oracle."""
+"""The step with its boundaries (vfx_k17_step_fused) against the separate
+boundary kernels of the unfused step: the stored populations agree bit for bit
+in FP64, FP32 and FP16 storage, over runs split into several step() calls.
+Stepper(fuse=True) takes the pressure boundary inside the collide-stream kernel
+and the others whole by their own kernels; a caller of Lattice.k17_step_fused
+may also hand it post-collision groups, which run after the step, with the
+entries no group takes left to apply_bc.  FP64 also against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -27,8 +28,26 @@ def _lattice(dims, solid, omega, storage, u_in):
     return lat
 
 
+def _calls(lat, bcs, chunks, any_mask=None):
+    """The run by FusedPlan's groups, handed to the call itself."""
+    plan = vfx.FusedPlan.build(lat, bcs)
+    even = True
+    for c in chunks:
+        for i in range(c):
+            lat.k17_step_fused(even, plan.post, plan.pre, apply_pre=i > 0, any_mask=any_mask)
+            for bc in plan.residual_post:
+                lat.apply_bc(bc, even)
+            even = not even
+            for bc in plan.residual_pre:
+                lat.apply_bc(bc, even)
+        if plan.pre is not None:
+            lat.apply_bc(plan.pre.bc, even)
+    return lat
+
+
 def _pair(dims, solid, omega, tables, storage, u_in, chunks, fuse_post=True):
-    """The same run unfused (one call) and fused (calls of `chunks` steps)."""
+    """The same run unfused (one call), fused (calls of `chunks` steps) and, with
+    fuse_post, by calls with post-collision groups."""
     a = _lattice(dims, solid, omega, storage, u_in)
     b = _lattice(dims, solid, omega, storage, u_in)
     sa = vfx.Stepper(a, "k17", geometry.boundary_conditions(tables))
@@ -38,6 +57,9 @@ def _pair(dims, solid, omega, tables, storage, u_in, chunks, fuse_post=True):
         sb.step(c)
     torch.cuda.synchronize()
     assert sa.even == sb.even
+    if fuse_post:
+        c = _lattice(dims, solid, omega, storage, u_in)
+        assert _same(a, _calls(c, geometry.boundary_conditions(tables), chunks))
     return a, b, sb
 
 
@@ -101,7 +123,8 @@ def test_outlet_on_a_wavefront_edge_runs_as_residual(cuda, storage):
 @pytest.mark.parametrize("storage", ("fp64", "fp32", "fp16"))
 def test_mixed_fused_and_residual_entries(cuda, storage):
     """A fluid node behind one wall link and solid inward neighbours of some
-    outlet nodes: those entries run in residual kernels, the rest fused."""
+    outlet nodes: no group takes those entries.  The stepper runs the wall
+    boundary whole, the calls split it."""
     print(f"[fused channel mixed split {storage}]", flush=True)
     ch = small_channel()
     nx, ny, nz = ch.dims
@@ -172,7 +195,7 @@ def test_no_groups_is_the_plain_step(cuda, storage):
 @pytest.mark.parametrize("storage", FORMS)
 @pytest.mark.parametrize("part", ("noslip", "velocity", "pressure"))
 def test_one_group(cuda, storage, part):
-    """Each boundary group of the channel fused alone."""
+    """Each boundary of the channel alone: the groups of a call in turn."""
     print(f"[fused {part} only {storage}]", flush=True)
     ch = small_channel()
     kind = {"noslip": 1, "velocity": 2, "pressure": 4}[part]
@@ -195,24 +218,22 @@ def test_fused_rejects_unsupported_lattices(cuda):
 
 
 def test_without_union_mask(cuda):
-    """any_mask NULL: every node looks its groups up itself; same result."""
-    print("[fused channel without union mask fp16]", flush=True)
+    """any_mask is accepted and not read: the union, none and an empty one."""
+    print("[fused channel union masks fp16]", flush=True)
     ch = small_channel()
-    a, b, st = _pair(ch.dims, ch.solid, ch.omega, ch.bcs, "fp16", ch.u_in, (5, 5))
-    c = _lattice(ch.dims, ch.solid, ch.omega, "fp16", ch.u_in)
-    sc = vfx.Stepper(c, "k17", geometry.boundary_conditions(ch.bcs), fuse=True)
-    sc.fused_plan().any_mask = None
-    sc.step(5)
-    sc.step(5)
-    torch.cuda.synchronize()
-    assert _same(a, c) and _same(b, c)
+    out = []
+    for mask in ("union", None, "empty"):
+        lat = _lattice(ch.dims, ch.solid, ch.omega, "fp16", ch.u_in)
+        bcs = geometry.boundary_conditions(ch.bcs)
+        u = vfx.FusedPlan.build(lat, bcs).any_mask
+        out.append(_calls(lat, bcs, (5, 5), u if mask == "union" else u * 0 if mask == "empty" else None))
+    assert _same(out[0], out[1]) and _same(out[0], out[2])
 
 
 @pytest.mark.parametrize("storage", FORMS)
 def test_slip_group(cuda, storage):
-    """The channel's walls and spheres as slip boundaries (kind 3) fused with
-    the inlet: slip marks its face axes in link order, so its nodes take the
-    per-node path also in wavefronts whose other groups go link-parallel."""
+    """The channel's walls and spheres as slip boundaries (kind 3) beside the
+    inlet, both as groups of the call: run in the order they are handed over."""
     print(f"[fused slip channel {storage}]", flush=True)
     ch = small_channel()
     tables = []
