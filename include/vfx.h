@@ -231,6 +231,9 @@ typedef struct vfx_bc {
     const void* vz;
     int32_t cpu_float_velocity; /* 1: wall term of VFX_BC_VELOCITY_BOUNCE_BACK rounded as VirtualFluids' CPU
                                    BoundaryConditions does (float velocity and sum, BoundaryConditions.h:195-262) */
+    int32_t single_links;      /* VFX_BC_VELOCITY_BOUNCE_BACK, sparse layout: 1: the caller knows that no node of the
+                                  list is its own neighbour along any axis (0: some may be; the links then run in
+                                  pairs, short lists take longer) */
     const void* rho;           /* real[n], VFX_BC_PRESSURE_NEQ: prescribed density deviation per boundary node (RhoBC) */
     const uint32_t* k_neighbor;/* VFX_BC_PRESSURE_NEQ / outflow: inward neighbour node of each boundary node */
     int32_t normal;            /* VFX_BC_PRESSURE_NEQ / outflow: outward direction of the boundary (e.g. 1 = dP00);

@@ -1,4 +1,4 @@
-"""The bounce-back kernel (one thread per pair of links) on lists whose length sits at the
+"""The bounce-back kernel (one thread per link or pair of links) on lists whose length sits at the
 edges of a wavefront and a workgroup, with links chosen at random: every element
 of the array against the formula, on the structured and the sparse layout, and
 the boundary set's one-thread-per-node form against the kernel bit for bit."""
@@ -93,6 +93,26 @@ def test_a_node_that_is_its_own_neighbour(cuda, axis, sparse):
         at = _at(nodes, INV[d], dims)
         ref[d, at] = f.reshape(27, n)[INV[d], at]
     assert np.array_equal(lat.f.cpu().numpy().reshape(27, n), ref)
+
+
+@pytest.mark.parametrize("storage", ["fp64", "fp32", "fp16"])
+@pytest.mark.parametrize("even", [True, False])
+def test_pairs_give_the_single_links_bytes(cuda, even, storage):
+    """A sparse list none of whose nodes is its own neighbour runs a thread per
+    link, any other a thread per pair: the same bytes."""
+    print(f"[bounce back single {even} {storage}]", flush=True)
+    nodes, q, u, f = _case(257, 5)
+    bc = vfx.BoundaryCondition(0, nodes, q, *u)
+    out = []
+    for single in (1, 0):
+        lat = _lattice(storage, True, f)
+        s, b = lat.struct(), lat._bc_struct(bc)
+        assert b.single_links == 1
+        b.single_links = single
+        C = vfx._lib.C
+        vfx.check(vfx.lib().vfx_bc_apply(C.byref(s), C.byref(b), int(even), None), "vfx_bc_apply")
+        out.append(lat.f.view(torch.uint8))
+    assert torch.equal(*out)
 
 
 @pytest.mark.parametrize("storage", ["fp64", "fp32", "fp16"])

@@ -103,6 +103,23 @@ def test_a_reader_may_change_the_lattice(library):
     assert omegas == pytest.approx([1.5, 1.51, 1.52, 1.53])
 
 
+@pytest.mark.parametrize("own,nodes,single", [(None, [3, 7], 1), (0, [3, 7], 1), (9, [3, 7], 1), (7, [3, 7], 0),
+                                              (5, [3, 7], 0)])
+def test_sparse_lists_say_when_no_node_is_its_own_neighbour(library, own, nodes, single):
+    """own: a node that is its own neighbour along y; a list whose node numbers
+    lie on one side of all such nodes holds none of them."""
+    n = 12
+    k = np.arange(n, dtype=np.uint32)
+    y = (k + 3) % n
+    if own is not None:
+        y[own] = own
+    lat = vfx.Lattice(storage="fp32", omega=1.5, neighbors=[(k + 1) % n, y, (k + 5) % n], fluid_nodes=k, device="cpu",
+                      regular_groups=False)
+    bc = vfx.BoundaryCondition(0, nodes, np.full((27, 2), 0.5), device="cpu")
+    assert lat._bc_struct(bc).single_links == single
+    assert vfx.Lattice((3, 4, 1), storage="fp32", omega=1.5, device="cpu")._bc_struct(bc).single_links == 0
+
+
 def test_plain_lattices_make_one_view(library, monkeypatch):
     lat = vfx.Lattice(DIMS, storage="fp32", omega=1.5, device="cpu")
     made = []

@@ -49,6 +49,7 @@ class VfxBC(C.Structure):
     _fields_ = [
         ("kind", C.c_int32), ("n", C.c_uint32), ("k", C.c_void_p), ("q27", C.c_void_p),
         ("vx", C.c_void_p), ("vy", C.c_void_p), ("vz", C.c_void_p), ("cpu_float_velocity", C.c_int32),
+        ("single_links", C.c_int32),
         ("rho", C.c_void_p), ("k_neighbor", C.c_void_p), ("normal", C.c_int32),
         ("pressure_correction_factor", C.c_double),
         ("wm_normal", C.c_void_p * 3), ("wm_exchange_velocity", C.c_void_p * 3), ("wm_wall_velocity", C.c_void_p * 3),

@@ -372,7 +372,7 @@ static vfx_status make_bcdev(const vfx_lattice* lat, const vfx::Lat& L, const vf
     } else if (bc->n && (!bc->k || !bc->q27)) {
         return fail(VFX_EINVAL, "bc.k / bc.q27 is NULL");
     }
-    B = vfx::BCDev{bc->n, bc->k, bc->q27, bc->vx, bc->vy, bc->vz, bc->cpu_float_velocity, lat->direct,
+    B = vfx::BCDev{bc->n, bc->k, bc->q27, bc->vx, bc->vy, bc->vz, bc->cpu_float_velocity, bc->single_links == 1, lat->direct,
                  lat->omega, bc->rho, bc->k_neighbor, bc->normal, bc->pressure_correction_factor,
                  {bc->wm_normal[0], bc->wm_normal[1], bc->wm_normal[2]},
                  {bc->wm_exchange_velocity[0], bc->wm_exchange_velocity[1], bc->wm_exchange_velocity[2]},

@@ -1088,6 +1088,7 @@ struct BCDev {
     const void* vy;
     const void* vz;
     int32_t cpu_float;
+    int32_t single_links;  // bounce-back, sparse: no node of the list is its own neighbour
     int32_t direct;
     double omega;          // interpolated kinds
     const void* rho;       // pressure: density deviation per boundary node
@@ -1249,9 +1250,14 @@ __device__ __forceinline__ void bb_links(const Lat& L, const BCDev& B, uint32_t 
         const int d = dir[j];
         // next step (parity !EVEN) reads direction e of node k from here
         const int e = inv(d);
-        if (on[j])
+        if (on[j]) {
             Storage<S, T>::st(plane<S>(L, slot(e, !EVEN)), kk[nbr(e)], bb_value<T>(d, f[j], ux, uy, uz, B.cpu_float),
                               L.st[weight_class(e)], L.ss[e]);
+            // keeps the branches of a switch over links apart: with their ends
+            // merged, the FMA of a half's store and its conversion (one
+            // instruction, one rounding) come apart and round twice
+            asm volatile("" ::"n"(dir[j]));
+        }
     }
 }
 template <typename S, bool EVEN>
@@ -1261,34 +1267,56 @@ __device__ __forceinline__ void bc_velocity_bb_entry(const Lat& L, const BCDev& 
         bb_links<S, EVEN, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, 18, 19, 20, 21, 22, 23, 24, 25, 26>(L, B, i);
 }
 
-// One thread per link and its opposite: blockIdx.y is the pair, so a wavefront
-// holds one pair of 64 boundary nodes and everything about its links is a
-// constant of the switch branch it takes.  The two stay in one thread because
-// they exchange the same two elements where a node is its own neighbour along
-// them (an axis of one node): loads first, then stores.  Any other element is
-// touched by one link only.  Lists are bound by latency: with the links of a
-// node one after another in one thread each waited for the one before (its
-// fraction, its population and its store, 26 round trips); here the chain is
-// fraction -> population -> store.  Long sparse lists add the neighbour indices
-// to it (up to three dependent loads) and read 26 fractions and 13 node numbers
-// a node, of which a third are walls.  MI355X, us
-// per launch: a thread for all links of a node, one after another, against one
-// per link, cavity 30^3 FP32 13.6 and 3.6, 64^3 FP64 17.5 and 6.2; one per link
-// against one per pair, launches back to back, 4.5 and 4.4, 5.9 and 5.5; 4 steps
-// with y and z walls and spheres of a 320x130x134 sparse box, FP16, 673 and 664.
-template <typename S, bool EVEN>
+// One thread per link (PAIRS: per link and its opposite): blockIdx.y is the
+// direction, so a wavefront holds one direction of 64 boundary nodes and
+// everything about the link is a constant of the switch branch it takes.  Lists
+// are bound by latency: with the links of a node one after another in one thread
+// each waited for the one before (its fraction, its population and its store, 26
+// round trips); here the chain is fraction -> population -> store, on the sparse
+// layout with up to three dependent loads of neighbour indices in between.
+// MI355X, us per launch, all links of a node one after another -> one per thread:
+// cavity 30^3 FP32 13.6 -> 3.6, 64^3 FP64 17.5 -> 6.2; 3, 7, 13 and 26 links per
+// thread: 30^3 4.3 / 4.7 / 5.8 / 7.3, 128^3 FP16 14.4 / 14.9 / 14.9 / 15.9
+// against 15.9.
+//
+// Where a node is its own neighbour along a link (an axis of one node), the link
+// and its opposite exchange the same two elements and must share a thread, loads
+// first; any other element is touched by one link only.  A structured box shows
+// that by its dims; on the sparse layout the caller says that no node of the list
+// is its own neighbour (single_links), otherwise pairs.  One link / one pair per thread, us per 6 steps: cavity 20^3
+// FP16 43 / 48, 66^3 FP64 190 / 187; sparse 62x58x56 FP16 85 / 87, 150x100x110
+// FP16 291 / 289, FP64 987 / 994 (one link that looks for its opposite's
+// neighbour itself: 87, 303, 1005).
+template <typename S, bool EVEN, bool PAIRS>
 __global__ void __launch_bounds__(256) k_bc_velocity_bb(Lat L, BCDev B)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= B.n) return;
+#define VFX_LINK(D) \
+    case D: bb_links<S, EVEN, D>(L, B, i); break;
 #define VFX_PAIR(Y, D) \
     case Y: bb_links<S, EVEN, D, inv(D)>(L, B, i); break;
-    switch (blockIdx.y) {
-        VFX_PAIR(0, dP00) VFX_PAIR(1, d0P0) VFX_PAIR(2, d00P) VFX_PAIR(3, dPP0) VFX_PAIR(4, dPM0) VFX_PAIR(5, dP0P)
-        VFX_PAIR(6, dP0M) VFX_PAIR(7, d0PP) VFX_PAIR(8, d0PM) VFX_PAIR(9, dPPP) VFX_PAIR(10, dPPM) VFX_PAIR(11, dPMP)
-        VFX_PAIR(12, dMPP)
-    }
+    if constexpr (PAIRS) switch (blockIdx.y) {
+            VFX_PAIR(0, dP00) VFX_PAIR(1, d0P0) VFX_PAIR(2, d00P) VFX_PAIR(3, dPP0) VFX_PAIR(4, dPM0) VFX_PAIR(5, dP0P)
+            VFX_PAIR(6, dP0M) VFX_PAIR(7, d0PP) VFX_PAIR(8, d0PM) VFX_PAIR(9, dPPP) VFX_PAIR(10, dPPM)
+            VFX_PAIR(11, dPMP) VFX_PAIR(12, dMPP)
+        }
+    else switch (blockIdx.y + 1) {
+            VFX_LINK(1) VFX_LINK(2) VFX_LINK(3) VFX_LINK(4) VFX_LINK(5) VFX_LINK(6) VFX_LINK(7) VFX_LINK(8) VFX_LINK(9)
+            VFX_LINK(10) VFX_LINK(11) VFX_LINK(12) VFX_LINK(13) VFX_LINK(14) VFX_LINK(15) VFX_LINK(16) VFX_LINK(17)
+            VFX_LINK(18) VFX_LINK(19) VFX_LINK(20) VFX_LINK(21) VFX_LINK(22) VFX_LINK(23) VFX_LINK(24) VFX_LINK(25)
+            VFX_LINK(26)
+        }
 #undef VFX_PAIR
+#undef VFX_LINK
+}
+template <typename S> hipError_t launch_velocity_bb(const Lat& L, const BCDev& B, bool even, hipStream_t st)
+{
+    const bool pairs = B.direct ? L.nx == 1 || L.ny == 1 || L.nz == 1 : !B.single_links;
+    auto* kernel = pairs ? (even ? k_bc_velocity_bb<S, true, true> : k_bc_velocity_bb<S, false, true>)
+                         : (even ? k_bc_velocity_bb<S, true, false> : k_bc_velocity_bb<S, false, false>);
+    hipLaunchKernelGGL(kernel, dim3((B.n + 255u) / 256u, pairs ? 13 : 26), dim3(256), 0, st, L, B);
+    return hipGetLastError();
 }
 
 // Interpolated bounce-back family (NoSlipInterpolatedCompressible.cu:44-378,
@@ -2708,10 +2736,7 @@ template <typename S> hipError_t launch_bc(const Lat& L, const BCDev& B, int kin
     if (B.n == 0) return hipSuccess;
     const dim3 g(grid_for(B.n, kBlock)), b(kBlock);
     switch (kind) {
-    case VFX_BC_VELOCITY_BOUNCE_BACK:
-        if (even) hipLaunchKernelGGL((k_bc_velocity_bb<S, true>), dim3(g.x, 13), b, 0, st, L, B);
-        else hipLaunchKernelGGL((k_bc_velocity_bb<S, false>), dim3(g.x, 13), b, 0, st, L, B);
-        break;
+    case VFX_BC_VELOCITY_BOUNCE_BACK: return launch_velocity_bb<S>(L, B, even, st);
     case VFX_BC_NOSLIP_INTERPOLATED:
         if (even) hipLaunchKernelGGL((k_bc_interp<S, true, VFX_BC_NOSLIP_INTERPOLATED>), g, b, 0, st, L, B);
         else hipLaunchKernelGGL((k_bc_interp<S, false, VFX_BC_NOSLIP_INTERPOLATED>), g, b, 0, st, L, B);

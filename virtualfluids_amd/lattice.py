@@ -112,6 +112,9 @@ class Lattice:
             if max(nbx.max(), nby.max(), nbz.max()) >= self.n_nodes:
                 raise ValueError("neighbour index out of range")
             self.nb = [torch.from_numpy(a.view(np.int32)).to(self.device) for a in (nbx, nby, nbz)]
+            own = np.arange(self.n_nodes, dtype=np.uint32)
+            own = np.flatnonzero((nbx == own) | (nby == own) | (nbz == own))
+            self.own_neighbors = (int(own[0]), int(own[-1])) if own.size else None
             if node_types is not None:
                 # VirtualFluids' typeOfGridNode: every node that is not
                 # GEO_SOLID (15) or GEO_VOID (16) collides
@@ -300,10 +303,19 @@ class Lattice:
         if bc.precursor is not None and bc.precursor.real != self._macro_dtype():
             raise ValueError("precursor weights and planes must have the lattice's arithmetic type")
 
+    def _bc_struct(self, bc: "BoundaryCondition") -> V.VfxBC:
+        b = bc.struct(self._macro_dtype())
+        if not self.direct and bc.n:
+            # nodes that are their own neighbour lie in this range of node numbers
+            # (a null node 0, say), or there are none
+            own = getattr(self, "own_neighbors", (0, self.n_nodes))
+            b.single_links = int(own is None or own[1] < bc.min_node or own[0] > bc.max_node)
+        return b
+
     def apply_bc(self, bc: "BoundaryCondition", even=True, stream=None):
         self._check_bc(bc)
         s = self.struct()
-        b = bc.struct(self._macro_dtype())
+        b = self._bc_struct(bc)
         V.check(V.lib().vfx_bc_apply(C.byref(s), C.byref(b), int(bool(even)), _stream(stream)), "vfx_bc_apply")
 
     def k17_step_fused(self, even, post=(), pre=None, apply_pre=False, any_mask=None, stream=None):
@@ -523,6 +535,7 @@ class BoundaryCondition:
         self.n = n
         dev = torch.device(device)
         self.max_node = int(nodes.max()) if n else -1
+        self.min_node = int(nodes.min()) if n else 0
         self.k = torch.from_numpy(nodes.view(np.int32)).to(dev)
         self.wm = None
         if self.kind in self.STRESS:
@@ -1020,7 +1033,7 @@ class Stepper:
                 lat.apply_bc(bc, even, stream=stream)
             return every_step
         lat._check_bc(bc)
-        b = bc.struct(lat._macro_dtype())
+        b = lat._bc_struct(bc)
         apply, st = V.lib().vfx_bc_apply, _stream(stream)
         args = C.byref(s), C.byref(b)
         return lambda even: V.check(apply(*args, int(even), st), "vfx_bc_apply")
