@@ -300,6 +300,22 @@ def test_capture_before_any_eager_step(cuda, merged):
     assert torch.equal(a.coarse.f, b.coarse.f) and torch.equal(a.fine.f, b.fine.f)
 
 
+def test_capture_with_the_outlet_inside_before_any_eager_step(cuda):
+    """The fused outlet's own tables are made with the stepper, not in the capture,
+    where an allocation may be refused."""
+    print("[refined capture first, fused outlet]", flush=True)
+    a, b = _cube_stepper_kw("fp32"), _cube_stepper_kw("fp32", fuse_outlet=True)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    before = torch.cuda.memory_allocated()
+    g = b.capture(2)
+    assert torch.cuda.memory_allocated() == before
+    b.replay(g, 2)
+    a.step(2)
+    torch.cuda.synchronize()
+    assert torch.equal(a.coarse.f, b.coarse.f) and torch.equal(a.fine.f, b.fine.f)
+
+
 @pytest.mark.parametrize("merged", [False, True])
 def test_autotuned_levels_give_the_same_bytes(cuda, merged):
     """RefinedStepper.autotune picks each level's launch shape and restores the

@@ -6,6 +6,7 @@ import pytest
 
 import virtualfluids_amd as vfx
 from tests.test_geometry import small_channel
+from tests.test_oracle_refinement import small_cube_case
 from virtualfluids_amd import _lib, geometry, lattice
 
 DIMS = (6, 5, 4)
@@ -168,3 +169,23 @@ def test_fused_steps_run_other_boundaries_whole(library, fuse_post):
     outlet = seen.pop()
     assert outlet.kind == 4 and outlet.n == next(b for b in bcs if b.pre_collision).n
     assert seen == [([], True, None)] + post + [([], True, None)] + post
+
+
+def test_plans_make_their_tables(monkeypatch):
+    """A step may be captured right after fused_plan() or a RefinedStepper with
+    fuse_outlet: the boundaries a plan splits off have their tables by then."""
+    ch = small_channel()
+    lat = vfx.Lattice(ch.dims, storage="fp32", omega=1.5, solid=ch.solid, device="cpu")
+    st = vfx.Stepper(lat, "k17", geometry.boundary_conditions(ch.bcs, device="cpu"), fuse=True)
+    st.fused_plan()
+    monkeypatch.setattr(vfx.FusedPlan, "build", None)
+    plan = st._plan(False)
+    assert lat._macro_dtype() in plan.pre.bc._dev
+    monkeypatch.undo()
+    case = small_cube_case()
+    r = vfx.RefinedStepper(case.nest, case.omega, storage="fp32", device="cpu", coarse_solid=case.coarse_solid,
+                           fine_solid=case.fine_solid, fuse_outlet=True,
+                           coarse_bcs=geometry.boundary_conditions(case.coarse_bcs, device="cpu"),
+                           fine_bcs=geometry.boundary_conditions(case.fine_bcs, device="cpu"))
+    parts = [r._plan_c.pre.bc] + r._plan_c.residual_pre + r._plan_c.residual_post
+    assert all(r.coarse._macro_dtype() in b._dev for b in parts)

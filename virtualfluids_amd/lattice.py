@@ -804,8 +804,9 @@ def fusable_post_entries(lattice, bc) -> np.ndarray:
 def fusable_pressure_entries(lattice, bc) -> np.ndarray:
     """Entries of a non-equilibrium pressure boundary on a face normal to +-x
     the kernel may apply itself: fluid node appearing once, inward neighbour
-    k -+ 1 in the same row and the same 64-node wavefront, fluid and no node of
-    the boundary.  All False when any neighbour is a boundary node."""
+    k -+ 1 in the same row, fluid and no node of the boundary, and x mod 64 != 0
+    (!= 63 for -x), which vfx_k17_step_fused asks for in every row length.  All
+    False when any neighbour is a boundary node."""
     n = bc.n
     if bc.kind != V.VFX_BC_PRESSURE_NEQ or bc.normal not in (1, 2) or n == 0:
         return np.zeros(n, dtype=bool)
@@ -990,6 +991,7 @@ class Stepper:
     _plan_key: tuple | None = field(default=None, init=False, repr=False)
 
     def fused_plan(self) -> FusedPlan:
+        self._plan(False)  # the steps' own: made here, so that they may be captured next
         return self._plan(self.fuse_post)
 
     def _plan(self, post) -> FusedPlan:
@@ -1004,7 +1006,9 @@ class Stepper:
         if self._plan_key != key:
             self._plans, self._plan_key = {}, key
         if post not in self._plans:
-            self._plans[post] = FusedPlan.build(lat, self.bcs, post=post)
+            plan = self._plans[post] = FusedPlan.build(lat, self.bcs, post=post)
+            for bc in ([plan.pre.bc] if plan.pre is not None else []) + plan.residual_pre:
+                bc.tables(lat._macro_dtype())
         return self._plans[post]
 
     def _prime(self, stream):

@@ -354,6 +354,8 @@ class RefinedStepper:
             self._plan_c = FusedPlan.build(self.coarse, self.coarse_bcs, post=False)
             if self._plan_c.pre is None:
                 raise ValueError("fuse_outlet: the coarse level has no pressure group the kernel can take")
+            for bc in [self._plan_c.pre.bc] + self._plan_c.residual_post + self._plan_c.residual_pre:
+                bc.tables(real)  # the plan's own parts of the boundaries
 
     def _setup_merged(self):
         """Fewer launches per coarse step (same values): the coarse step and the
