@@ -320,8 +320,9 @@ typedef struct vfx_fused_bc {
  *    the step in this order, by the kernels of vfx_bc_apply (inside the step
  *    they cost more than their own launches);
  *  - pre (or NULL): VFX_BC_PRESSURE_NEQ with normal dP00 (dM00) whose every
- *    entry has k_neighbor = k - 1 (k + 1) in the same wavefront of 64 nodes,
- *    i.e. x mod 64 != 0 (!= 63): the replacement vfx_bc_apply makes after the
+ *    entry has k_neighbor = k - 1 (k + 1), a fluid node, and x mod 64 != 0
+ *    (!= 63; in rows of a multiple of 64 nodes the pair is then in one
+ *    wavefront): the replacement vfx_bc_apply makes after the
  *    previous step's parity flip is made inside this step, from the
  *    neighbour's populations the neighbouring lane gathers, which spares the
  *    cache lines a kernel of its own reads again.  apply_pre: 0 on the first

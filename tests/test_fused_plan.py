@@ -49,8 +49,8 @@ def test_group_rejects_unsorted_or_repeated_nodes():
 
 
 def test_channel_entries_are_all_fusable():
-    """Every wall link of the channel ends in a solid node and the outlet's
-    inward neighbour sits in the same 64-node wavefront: all entries fuse."""
+    """Every wall link of the channel ends in a solid node and the outlet is not
+    at x mod 64 = 0: all entries fuse."""
     ch = small_channel()
     lat = _lat(ch)
     bcs = _bcs(ch)

@@ -110,8 +110,8 @@ def test_channel_fused_fp64_matches_oracle(cuda):
 
 @pytest.mark.parametrize("storage", ("fp64", "fp16"))
 def test_outlet_on_a_wavefront_edge_runs_as_residual(cuda, storage):
-    """Outlet at x = 64: the inward neighbour x = 63 sits in the previous
-    wavefront, so the pressure entries stay in a kernel of their own."""
+    """Outlet at x = 64: the call takes no entry with x mod 64 = 0, so the
+    pressure entries stay in a kernel of their own."""
     print(f"[fused channel outlet x=64 {storage}]", flush=True)
     ch = geometry.spheres_in_channel(dims=(66, 20, 18), n_spheres=3, r_range=(2.5, 4.0), x_clear=(8, 10))
     a, b, st = _pair(ch.dims, ch.solid, ch.omega, ch.bcs, storage, ch.u_in, (5, 9))

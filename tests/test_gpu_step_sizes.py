@@ -70,18 +70,20 @@ def test_fp16_models_reduced_form_equals_the_reference_order(cuda, model, sparse
 
 
 @pytest.mark.parametrize("model", ["smagorinsky", "qr", "amd"])
-@pytest.mark.parametrize("dims", [(37, 11, 8), (65, 16, 9)])
-def test_fp16_models_write_the_reference_orders_density_and_velocity(cuda, model, dims):
+@pytest.mark.parametrize("dims,body_force", [((37, 11, 8), False), ((65, 16, 9), False), ((37, 11, 8), True)])
+def test_fp16_models_write_the_reference_orders_density_and_velocity(cuda, model, dims, body_force):
     """The 32-bit fields the collision writes, and the viscosity the AMD kernel
     forms from them, are the same bits in the default and the "plain" variant."""
-    print(f"[fp16 fields {model} {dims}]", flush=True)
+    print(f"[fp16 fields {model} {dims} {body_force}]", flush=True)
     n = int(np.prod(dims))
     out = []
     for variant in ("default", "plain"):
         lat = vfx.Lattice(dims, storage="fp16", omega=1.95, turbulence=model, sgs_constant=0.2, variant=variant)
         lat.init_equilibrium(*cases.random_flow(dims, seed=9))
         lat.nut.copy_(torch.from_numpy(1e-3 * (1.0 + np.sin(np.arange(n)))).to(lat.nut.dtype))
-        lat.collide_stream("k17", True, write_macro=True)
+        if body_force:
+            lat.set_body_force(1e-4 * np.sin(np.arange(n)), 1e-4, -1e-4 * np.cos(np.arange(n)), forces=(1e-5, 0.0, 0.0))
+        lat.collide_stream("k17", True, write_macro=True, apply_body_force=body_force)
         fields = list(lat.macro)
         if model == "amd":
             lat.turbulent_viscosity_amd()

@@ -1283,10 +1283,10 @@ __device__ __forceinline__ void bc_velocity_bb_entry(const Lat& L, const BCDev& 
 // and its opposite exchange the same two elements and must share a thread, loads
 // first; any other element is touched by one link only.  A structured box shows
 // that by its dims; on the sparse layout the caller says that no node of the list
-// is its own neighbour (single_links), otherwise pairs.  One link / one pair per thread, us per 6 steps: cavity 20^3
-// FP16 43 / 48, 66^3 FP64 190 / 187; sparse 62x58x56 FP16 85 / 87, 150x100x110
-// FP16 291 / 289, FP64 987 / 994 (one link that looks for its opposite's
-// neighbour itself: 87, 303, 1005).
+// is its own neighbour (single_links), otherwise pairs.  One link / one pair per
+// thread, us per 6 steps: cavity 20^3 FP16 43 / 48, 66^3 FP64 190 / 187; sparse
+// 62x58x56 FP16 85 / 87, 150x100x110 FP16 291 / 289, FP64 987 / 994 (one link that
+// looks for its opposite's neighbour itself: 87, 303, 1005).
 template <typename S, bool EVEN, bool PAIRS>
 __global__ void __launch_bounds__(256) k_bc_velocity_bb(Lat L, BCDev B)
 {
