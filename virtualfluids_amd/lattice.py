@@ -112,9 +112,9 @@ class Lattice:
             if max(nbx.max(), nby.max(), nbz.max()) >= self.n_nodes:
                 raise ValueError("neighbour index out of range")
             self.nb = [torch.from_numpy(a.view(np.int32)).to(self.device) for a in (nbx, nby, nbz)]
-            own = np.arange(self.n_nodes, dtype=np.uint32)
-            own = np.flatnonzero((nbx == own) | (nby == own) | (nbz == own))
-            self.own_neighbors = (int(own[0]), int(own[-1])) if own.size else None
+            own = torch.arange(self.n_nodes, dtype=torch.int32, device=self.device)
+            own = torch.nonzero((self.nb[0] == own) | (self.nb[1] == own) | (self.nb[2] == own)).view(-1)
+            self.own_neighbors = tuple(own[[0, -1]].tolist()) if own.numel() else None
             if node_types is not None:
                 # VirtualFluids' typeOfGridNode: every node that is not
                 # GEO_SOLID (15) or GEO_VOID (16) collides
