@@ -957,7 +957,11 @@ _BC_TABLES = {n: BoundaryCondition.__dict__[n] for n in ("struct", "tables")}
 
 
 def _as_defined(obj, methods) -> bool:
-    return all(getattr(type(obj), n, None) is f and n not in getattr(obj, "__dict__", ()) for n, f in methods.items())
+    cls, own = type(obj), getattr(obj, "__dict__", ())
+    for name, method in methods.items():
+        if getattr(cls, name, None) is not method or name in own:
+            return False
+    return True
 
 
 @dataclass
@@ -1065,6 +1069,24 @@ class Stepper:
         if plan.pre is not None:
             lat.apply_bc(plan.pre.bc, self.even, stream=stream)
 
+    def _step_each(self, n, write_macro, stream):
+        """step(n) through the lattice's own launches, every step."""
+        lat = self.lattice
+        order = sorted(self.bcs, key=lambda b: b.kind in BoundaryCondition.PRECURSOR)
+        post = [self._bc_call(b, None, stream) for b in order if not b.pre_collision]
+        pre = [self._bc_call(b, None, stream) for b in self.bcs if b.pre_collision]
+        for _ in range(n):
+            lat.collide_stream(self.collision, self.even, write_macro=write_macro, stream=stream,
+                               apply_body_force=self.apply_body_force)
+            for run in post:
+                run(self.even)
+            self.t += 1
+            self.even = not self.even
+            if self.collision == "k17" and getattr(lat, "turbulence", "none") == "amd":
+                lat.turbulent_viscosity_amd(stream=stream)
+            for run in pre:
+                run(self.even)
+
     def step(self, n=1, stream=None):
         if self.fuse:
             return self._step_fused(n, stream)
@@ -1074,39 +1096,26 @@ class Stepper:
         lat = self.lattice
         # wall models sample the velocities the collision writes
         write_macro = any(getattr(b, "wm", None) is not None for b in self.bcs)
+        if not self._one_view():
+            return self._step_each(n, write_macro, stream)
+        tmpl = lat._template(write_macro, self.apply_body_force)  # makes the arrays the view holds
         # the lattice and its tables are handed over once per call, not once per
         # launch: a small lattice's step takes less time than making the views
-        s = None
-        if self._one_view():
-            tmpl = lat._template(write_macro, self.apply_body_force)  # makes the arrays the view holds
-            s = lat.struct()
+        s = lat.struct()
         # precursor inflows run last among the post-collision conditions (UpdateGrid27.cpp:252)
         order = sorted(self.bcs, key=lambda b: b.kind in BoundaryCondition.PRECURSOR)
         post = [self._bc_call(b, s, stream) for b in order if not b.pre_collision]
         pre = [self._bc_call(b, s, stream) for b in self.bcs if b.pre_collision]
-        if s is None:
-            def collide(even):
-                lat.collide_stream(self.collision, even, write_macro=write_macro, stream=stream,
-                                   apply_body_force=self.apply_body_force)
-
-            def viscosity():
-                lat.turbulent_viscosity_amd(stream=stream)
-        else:
-            L, st, view, coll = V.lib(), _stream(stream), C.byref(s), COLLISION[self.collision]
-
-            def collide(even):
-                V.check(L.vfx_collide_stream(view, coll, int(even), tmpl, st), "vfx_collide_stream")
-
-            def viscosity():
-                V.check(L.vfx_turbulent_viscosity_amd(view, st), "vfx_turbulent_viscosity_amd")
+        L, st, view, coll = V.lib(), _stream(stream), C.byref(s), COLLISION[self.collision]
+        amd = self.collision == "k17" and getattr(lat, "turbulence", "none") == "amd"
         for _ in range(n):
-            collide(self.even)
+            V.check(L.vfx_collide_stream(view, coll, int(self.even), tmpl, st), "vfx_collide_stream")
             for run in post:
                 run(self.even)
             self.t += 1
             self.even = not self.even
-            if self.collision == "k17" and getattr(lat, "turbulence", "none") == "amd":
-                viscosity()
+            if amd:
+                V.check(L.vfx_turbulent_viscosity_amd(view, st), "vfx_turbulent_viscosity_amd")
             for run in pre:
                 run(self.even)
 
