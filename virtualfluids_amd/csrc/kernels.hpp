@@ -904,15 +904,15 @@ template <int NV> __device__ __forceinline__ void block_sum(double (&v)[NV])
 }
 
 // per node: drho, jx, jy, jz (mass deviation and momentum of the pre-collision state)
-template <typename S, bool EVEN>
-__global__ void __launch_bounds__(kRedBlock) k_reduce_mass(Lat L, int direct, double* partial)
+template <typename S, bool EVEN, bool DIRECT>
+__global__ void __launch_bounds__(kRedBlock) k_reduce_mass(Lat L, double* partial)
 {
     using T = typename Compute<S>::T;
     double acc[4] = {0, 0, 0, 0};
     for (int j = 0; j < kRedPerThread; ++j) {
         const uint64_t i = (uint64_t)blockIdx.x * kRedChunk + (uint64_t)j * kRedBlock + threadIdx.x;
         uint32_t kk[8];
-        if (!NodeIter::get(L, i, kk, direct)) continue;
+        if (!NodeIter::get(L, i, kk, DIRECT)) continue;
         T m[27];
         gather<S, T, EVEN>(L, kk, m);
         double r, jx, jy, jz;
@@ -2715,8 +2715,9 @@ template <typename S> hipError_t launch_reduce_mass(const Lat& L, int direct, bo
 {
     const uint64_t n = node_items(L, direct);
     const uint32_t nb = reduce_blocks(n ? n : 1);
-    if (even) hipLaunchKernelGGL((k_reduce_mass<S, true>), dim3(nb), dim3(kRedBlock), 0, st, L, direct, ws);
-    else hipLaunchKernelGGL((k_reduce_mass<S, false>), dim3(nb), dim3(kRedBlock), 0, st, L, direct, ws);
+    auto* kernel = direct ? (even ? k_reduce_mass<S, true, true> : k_reduce_mass<S, false, true>)
+                          : (even ? k_reduce_mass<S, true, false> : k_reduce_mass<S, false, false>);
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(kRedBlock), 0, st, L, ws);
     hipLaunchKernelGGL((k_reduce_finish<4>), dim3(1), dim3(kRedBlock), 0, st, ws, nb, out);
     return hipGetLastError();
 }
