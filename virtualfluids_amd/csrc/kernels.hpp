@@ -2732,10 +2732,20 @@ template <typename S> hipError_t launch_stats(const Lat& L, int direct, bool eve
     return hipGetLastError();
 }
 
+// One thread per boundary node.  A node of a face normal to x touches a cache
+// line per element, and those of a workgroup queue at one CU: lists that leave
+// CUs idle with workgroups of 256 (below 256 of them) run workgroups of 64.
+// MI355X, us per launch, workgroups of 256 / 64: interpolated inlet of 2784 nodes
+// 8.4 / 5.6, 5304 12.0 / 6.6, 8836 12.3 / 7.9, 20164 16.1 / 15.8, 64516 53 / 53;
+// pressure outlet of 5304 12.4 / 5.7, 8836 13.0 / 7.0, 20164 16.9 / 16.3; no-slip
+// walls of 22284 6.3 / 5.7, 48254 6.5 / 6.1, 97214 7.0 / 8.1, 518878 20 / 25 (FP32;
+// 64516 and 518878 FP16).  Channel 96x60x50 FP32 per step, outlet in the step:
+// 37.6 -> 30.2 (33.2 with the interpolated kinds in the step as well).
 template <typename S> hipError_t launch_bc(const Lat& L, const BCDev& B, int kind, bool even, hipStream_t st)
 {
     if (B.n == 0) return hipSuccess;
-    const dim3 g(grid_for(B.n, kBlock)), b(kBlock);
+    const unsigned w = B.n < 256u * kBlock ? 64u : kBlock;
+    const dim3 g(grid_for(B.n, w)), b(w);
     switch (kind) {
     case VFX_BC_VELOCITY_BOUNCE_BACK: return launch_velocity_bb<S>(L, B, even, st);
     case VFX_BC_NOSLIP_INTERPOLATED:
