@@ -1973,9 +1973,10 @@ __device__ __forceinline__ void fused_pressure(const Lat& L, const FusedGroup& G
 // populations, the entry while they arrive (after them: 150 us).  A boundary
 // node whose neighbour is in another wavefront (lane 0, or 63 for -x) is left to
 // k_bc_pressure_edge, launched before where the list has one.  MI355X, us per
-// step, FP16: channel 288x144x144 143 against 129 + 33 for the plain step and
-// k_bc_pressure (160 in turn), 230x130x120 with 472 of 15104 entries in the edge
-// launch 81 + 6.3 against 70 + 16.
+// step, with the outlet in the step / apart / without: 288x144x144 FP16 142 / 150 /
+// 128, FP32 256 / 293 / 256, FP64 524 / 582 / 511; 512x256x256 FP16 754 / 812 / 722,
+// FP64 2868 / 2990 / 2785; 96x60x50 FP16 15.7 / 20.1 / 12.0; 230x130x120, 472 of
+// 15104 entries in the edge launch (6.3), FP64 330 / 352 / 314, FP16 90 / 81 / 69.
 template <typename S, bool EVEN>
 __global__ void __launch_bounds__(256) k_step_pre(Lat L, Rates<typename Compute<S>::T> R, FusedGroup gp)
 {
